@@ -10,12 +10,14 @@ import re
 from pathlib import Path
 
 import torch
+from torch.autograd import forward_ad
 
 _PKG = Path(__file__).resolve().parent
 LIB_PATH = _PKG / "libhilberta_hip.so"
 HEADER = _PKG.parent / "include" / "hilberta_hip.h"
 
 HB_EINVAL = 1
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 _c_int, _c_i64, _c_f32, _p = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
 
@@ -53,6 +55,7 @@ SIGNATURES = {
         [_p, _p, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_int,
          _c_int, _c_int, _c_int, _p, _c_f32, _p, _p, _p, _c_i64, _c_i64, _c_i64, _p],
     ),
+    "hb_rotary_tables": (_c_int, [_p, _c_i64, ctypes.c_double, _p, _p, _p, _p]),
     "hb_adaln_modulate": (
         _c_int,
         [_c_int, _c_int, _c_int, _c_int, _c_f32, _p, _c_i64, _c_i64, _p, _c_i64, _c_i64, _p, _c_i64,
@@ -148,6 +151,20 @@ def check(rc: int, name: str) -> None:
 def stream_ptr(device) -> int:
     """Raw hipStream_t of torch's current stream on ``device``."""
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def is_plain(*tensors) -> bool:
+    """True for ordinary device tensors outside any transform: no subclass (fake tensors), no
+    dispatch or function mode, tracing or torch.func level, no forward- or reverse-mode gradient.
+    Calls that composed torch operations also serve take their fused kernel only then."""
+    if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or forward_ad._current_level >= 0 or torch.jit.is_tracing()
+            or torch.compiler.is_compiling()):
+        return False
+    grad = torch.is_grad_enabled()
+    return all(type(t) in _PLAIN_TYPES and t.is_cuda and not (grad and t.requires_grad)
+               for t in tensors)
 
 
 def require_gpu(*tensors) -> None:

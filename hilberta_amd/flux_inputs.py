@@ -15,6 +15,7 @@ in the order the tokens are stored, e.g. after the persistent Hilbert permutatio
 from __future__ import annotations
 
 import ctypes
+import math
 
 import torch
 
@@ -24,6 +25,8 @@ HEAD_DIM = 128
 THETA = 10000
 AXES_DIM = (16, 56, 56)
 _DTYPES = {torch.bfloat16: 0, torch.float16: 1}
+# position id types of the one-launch rotary tables (converted to float32, as composed)
+_ID_DTYPES = (torch.float32, torch.bfloat16, torch.float16, torch.float64, torch.int64, torch.int32)
 
 
 def rotary_tables(ids, theta=THETA, axes_dim=AXES_DIM):
@@ -31,6 +34,9 @@ def rotary_tables(ids, theta=THETA, axes_dim=AXES_DIM):
     angles pos * theta^(-2j/d) per axis, each value repeated for the pair, axes concatenated)."""
     if ids.ndim != 2 or ids.shape[1] != len(axes_dim) or sum(axes_dim) != HEAD_DIM:
         raise ValueError("ids must be [N, 3] and the axes must add up to 128")
+    if (_lib.is_plain(ids) and ids.dtype in _ID_DTYPES and type(theta) in (int, float)
+            and 0 < theta < math.inf and all(type(d) is int and d >= 0 and d % 2 == 0 for d in axes_dim)):
+        return _rotary_tables_hip(ids, float(theta), axes_dim)
     pos = ids.to(torch.float32).to(torch.float64)
     cos, sin = [], []
     for axis, dim in enumerate(axes_dim):
@@ -40,6 +46,17 @@ def rotary_tables(ids, theta=THETA, axes_dim=AXES_DIM):
         sin.append(angles.sin().repeat_interleave(2, dim=1))
     return (torch.cat(cos, 1).to(torch.float32).contiguous(),
             torch.cat(sin, 1).to(torch.float32).contiguous())
+
+
+def _rotary_tables_hip(ids, theta, axes_dim):
+    """rotary_tables of plain device ids in one launch (csrc/rope.hip)."""
+    pos = ids.detach().to(torch.float32).contiguous()
+    out = torch.empty(2, ids.shape[0], HEAD_DIM, dtype=torch.float32, device=ids.device)
+    with torch.cuda.device(ids.device):
+        rc = _lib.load().hb_rotary_tables(pos.data_ptr(), pos.shape[0], theta, (ctypes.c_int32 * 3)(*axes_dim),
+                                          out[0].data_ptr(), out[1].data_ptr(), _lib.stream_ptr(ids.device))
+    _lib.check(rc, "hb_rotary_tables")
+    return out[0], out[1]
 
 
 def _rows(x, name):

@@ -149,6 +149,15 @@ int hb_qk_prep(const void* src_text, const void* src_image, int64_t text_batch_s
                void* out, int64_t out_plane_stride, int64_t out_batch_stride,
                int64_t out_row_stride, hb_stream_t stream);
 
+/* Rotary tables of FLUX position ids (diffusers 0.36.0 FluxPosEmbed, inside the transformer that
+ * reference hilberta/flux_adapter.py wraps; its image ids are permuted at :210-212):
+ *   cos[t, 2j..2j+1] / sin[t, 2j..2j+1] = cos / sin of ids[t, axis] * theta^(-2i / axes_dim[axis])
+ * for pair i of each of the three axes, axes concatenated, angles in float64 and rounded to fp32.
+ * ids is fp32 [tokens, 3]; cos and sin fp32 [tokens, 128], 8-byte aligned; axes_dim is a host
+ * array of three even sizes adding up to 128. */
+int hb_rotary_tables(const float* ids, int64_t tokens, double theta, const int32_t* axes_dim,
+                     float* cos, float* sin, hb_stream_t stream);
+
 /* Gated residual update + AdaLN modulation, one pass per row (FLUX blocks).  For each of
  * batch x rows rows of `hidden` values (row i of batch b at base + b*batch_stride + i*row_stride):
  *   r = x + gate[b] * y            (skipped when y is NULL: r = x)
