@@ -56,6 +56,10 @@ SIGNATURES = {
          _c_int, _c_int, _c_int, _p, _c_f32, _p, _p, _p, _c_i64, _c_i64, _c_i64, _p],
     ),
     "hb_rotary_tables": (_c_int, [_p, _c_i64, ctypes.c_double, _p, _p, _p, _p]),
+    "hb_linear_rows": (
+        _c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _p, _p, _p, _p, _p, _p, _p, _p],
+    ),
+    "hb_sinusoid_rows": (_c_int, [_p, _p, _c_int, _c_int, _c_int, _p, _p]),
     "hb_adaln_modulate": (
         _c_int,
         [_c_int, _c_int, _c_int, _c_int, _c_f32, _p, _c_i64, _c_i64, _p, _c_i64, _c_i64, _p, _c_i64,

@@ -1,0 +1,112 @@
+"""Linear layers of a few rows: the FLUX conditioning path in streamed HIP launches (csrc/cond.hip).
+
+``linear_layers`` applies many layers to the same rows (every block's AdaLN modulation, diffusers
+0.36.0 AdaLayerNormZero and its kin); ``embed`` is CombinedTimestepGuidanceTextProjEmbeddings: the
+sinusoidal timestep and guidance embeddings and the pooled text, each through a SiLU MLP, summed.
+Both return what the separate torch calls return up to the order of each fp32 sum.  Rows, sizes or
+types the kernels do not take (more than eight rows, depths that are no multiple of 8, other than
+bf16 / fp16, traced or differentiated inputs) run as those torch calls.
+"""
+
+from __future__ import annotations
+
+import ctypes
+import math
+
+import torch
+import torch.nn.functional as F
+
+from . import _lib
+
+MAX_ROWS = 8       # input rows per launch (hb_linear_rows)
+MAX_LAYERS = 64    # layers per launch
+_DTYPES = {torch.bfloat16: 0, torch.float16: 1}
+
+
+def _takes(x, layers):
+    """Whether hb_linear_rows takes rows ``x`` through each (weight, bias) of ``layers``."""
+    if x.ndim != 2 or not 1 <= x.shape[0] <= MAX_ROWS or x.dtype not in _DTYPES or x.shape[1] % 8:
+        return False
+    if x.shape[1] == 0 or x.stride(1) != 1 or x.stride(0) % 8 or not 0 <= x.stride(0) < 2**31 or x.data_ptr() % 16:
+        return False
+    for w, b in layers:
+        if w.ndim != 2 or w.shape[1] != x.shape[1] or not w.shape[0] or not w.is_contiguous() or w.data_ptr() % 16:
+            return False
+        if b is not None and (b.shape != w.shape[:1] or not b.is_contiguous()):
+            return False
+        if any(t is not None and (t.dtype != x.dtype or t.device != x.device) for t in (w, b)):
+            return False
+    return _lib.is_plain(x, *(t for layer in layers for t in layer if t is not None))
+
+
+def _launch(xs, layers, outs, *, sum=1, silu=False):
+    """outs[o] = sum over s of layers[o * sum + s] applied to xs[o * sum + s], in few launches."""
+    x0 = xs[0]
+    per = MAX_LAYERS // sum
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    with torch.cuda.device(x0.device):
+        for lo in range(0, len(outs), per):
+            o = outs[lo:lo + per]
+            x, la = xs[lo * sum:(lo + per) * sum], layers[lo * sum:(lo + per) * sum]
+            m, pointers = len(x), ctypes.c_void_p * len(x)
+            rc = _lib.load().hb_linear_rows(
+                len(o), sum, x0.shape[0], _DTYPES[x0.dtype], int(silu), pointers(*[t.data_ptr() for t in x]),
+                (ctypes.c_int64 * m)(*[t.stride(0) for t in x]), pointers(*[w.data_ptr() for w, _ in la]),
+                pointers(*[ptr(b) for _, b in la]), (ctypes.c_void_p * len(o))(*[t.data_ptr() for t in o]),
+                (ctypes.c_int32 * len(o))(*[t.shape[1] for t in o]),
+                (ctypes.c_int32 * m)(*[t.shape[1] for t in x]), _lib.stream_ptr(x0.device))
+            _lib.check(rc, "hb_linear_rows")
+    return outs
+
+
+def linear_layers(x, layers):
+    """[F.linear(x, weight, bias) for weight, bias in layers] for rows x [B, K]."""
+    if not layers or not _takes(x, layers):
+        return [F.linear(x, w, b) for w, b in layers]
+    return _launch([x] * len(layers), layers, [x.new_empty(x.shape[0], w.shape[0]) for w, _ in layers])
+
+
+def timestep_projection(t, dim=256):
+    """diffusers get_timestep_embedding(flip_sin_to_cos=True, downscale_freq_shift=0): [cos | sin]
+    of t * 10000^(-j/half)."""
+    half = dim // 2
+    freqs = torch.exp(-math.log(10000) * torch.arange(half, dtype=torch.float32, device=t.device) / half)
+    angles = t[:, None].float() * freqs[None, :]
+    return torch.cat([angles.cos(), angles.sin()], dim=-1)
+
+
+def _mlp(x, layers):
+    (w1, b1), (w2, b2) = layers
+    return F.linear(F.silu(F.linear(x, w1, b1)), w2, b2)
+
+
+def embed(scalars, scalar_mlps, pooled, pooled_mlp, dim, *, silu=False):
+    """Sum over ``scalars`` (timestep, guidance: [B] in the model's type) of their MLP applied to
+    the [cos | sin] embedding of 1000 times the scalar, plus ``pooled_mlp`` of ``pooled`` [B, K];
+    its SiLU with ``silu``.  An MLP is two (weight, bias) layers with a SiLU between."""
+    mlps = [*scalar_mlps, pooled_mlp]
+    B = pooled.shape[0] if pooled.ndim == 2 else 0
+    first, second = [m[0] for m in mlps], [m[1] for m in mlps]
+    hidden = [w.shape[0] for w, _ in first]
+    if (1 <= len(scalars) <= 2 and dim % 8 == 0 and _takes(pooled, first[-1:]) and _lib.is_plain(*scalars)
+            and all(t.shape == (B,) and t.is_contiguous() and t.dtype == pooled.dtype
+                    and t.device == pooled.device for t in scalars)):
+        waves = pooled.new_empty(len(scalars), B, dim)
+        h = [pooled.new_empty(B, n) for n in hidden]
+        if (all(_takes(x, [layer]) for x, layer in zip(waves, first)) and
+                all(_takes(x, [layer]) for x, layer in zip(h, second)) and
+                len({w.shape[0] for w, _ in second}) == 1):
+            with torch.cuda.device(pooled.device):
+                rc = _lib.load().hb_sinusoid_rows(
+                    scalars[0].data_ptr(), scalars[1].data_ptr() if len(scalars) == 2 else None, B, dim,
+                    _DTYPES[pooled.dtype], waves.data_ptr(), _lib.stream_ptr(pooled.device))
+            _lib.check(rc, "hb_sinusoid_rows")
+            _launch([*waves, pooled], first, h, silu=True)
+            out = pooled.new_empty(B, second[0][0].shape[0])
+            return _launch(h, second, [out], sum=len(mlps), silu=silu)[0]
+    total = None
+    for t, mlp in zip(scalars, scalar_mlps):
+        y = _mlp(timestep_projection(t * 1000, dim).to(pooled.dtype), mlp)
+        total = y if total is None else total + y
+    total = total + _mlp(pooled, pooled_mlp)
+    return F.silu(total) if silu else total

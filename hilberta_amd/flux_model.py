@@ -41,6 +41,7 @@ from dataclasses import dataclass
 import torch
 import torch.nn.functional as F
 
+from .flux_cond import embed, linear_layers, timestep_projection  # noqa: F401
 from .flux_inputs import qk_prep_pair, rotary_tables
 from .flux_norm import adaln_modulate
 from .layout import index_select_rows
@@ -102,20 +103,6 @@ class _Init:
 
     def mlp(self, fan_in, hidden):
         return self.linear(hidden, fan_in), self.linear(hidden, hidden)
-
-
-def timestep_projection(t, dim=256):
-    """diffusers get_timestep_embedding(flip_sin_to_cos=True, downscale_freq_shift=0): [cos | sin]
-    of t * 10000^(-j/half)."""
-    half = dim // 2
-    freqs = torch.exp(-math.log(10000) * torch.arange(half, dtype=torch.float32, device=t.device) / half)
-    angles = t[:, None].float() * freqs[None, :]
-    return torch.cat([angles.cos(), angles.sin()], dim=-1)
-
-
-def _mlp(x, layers):
-    (w1, b1), (w2, b2) = layers
-    return F.linear(F.silu(F.linear(x, w1, b1)), w2, b2)
 
 
 class NativeAttention:
@@ -242,7 +229,7 @@ class FluxTransformer:
     [B, N, 3C] buffer (V is read from it in place), Q and K are normalised and rotated by one
     qk_prep_pair launch, every gated residual add is fused with the following AdaLN modulation
     (flux_norm.adaln_modulate; all blocks' modulation vectors depend only on the timestep
-    embedding and are computed up front), the MLP GELU runs in the GEMM epilogue, and the single
+    embedding and are computed up front, flux_cond.linear_layers), the MLP GELU runs in the GEMM epilogue, and the single
     blocks' output projection over [attention | mlp] is two accumulating GEMMs instead of a
     concatenation.
     """
@@ -307,10 +294,11 @@ class FluxTransformer:
 
     def _modulations(self, silu_t):
         """Every block's AdaLN vectors (they depend on the timestep embedding only)."""
-        double = [(F.linear(silu_t, *w["mod_x"]).chunk(6, dim=1), F.linear(silu_t, *w["mod_c"]).chunk(6, dim=1))
-                  for w in self.double]
-        single = [F.linear(silu_t, *w["mod"]).chunk(3, dim=1) for w in self.single]
-        scale, shift = F.linear(silu_t, *self.norm_out).chunk(2, dim=1)   # AdaLayerNormContinuous order
+        out = iter(linear_layers(silu_t, [w[m] for w in self.double for m in ("mod_x", "mod_c")]
+                                 + [w["mod"] for w in self.single] + [self.norm_out]))
+        double = [(next(out).chunk(6, dim=1), next(out).chunk(6, dim=1)) for _ in self.double]
+        single = [next(out).chunk(3, dim=1) for _ in self.single]
+        scale, shift = next(out).chunk(2, dim=1)   # AdaLayerNormContinuous order
         return double, single, (shift, scale)
 
     def _double_block(self, w, mods, x, xn, c, cn, cos, sin, attention, layer, next_mods, joint_out):
@@ -387,14 +375,15 @@ class FluxTransformer:
         return None, adaln_modulate(h[:, T:], shift, scale, y=p[:, T:], gate=gate, eps=s.eps)
 
     # ------------------------------------------------------------------ forward
-    def temb(self, timestep, guidance, pooled):
-        s = self.shape
-        t = timestep.to(self.dtype) * 1000
-        emb = _mlp(timestep_projection(t, s.timestep_dim).to(self.dtype), self.time_embedder)
+    def temb(self, timestep, guidance, pooled, *, silu=False):
+        """Summed timestep, guidance and pooled-text embeddings [B, hidden]; with ``silu`` their
+        SiLU, the input of every modulation."""
+        scalars, mlps = [timestep.to(self.dtype)], [self.time_embedder]
         if self.guidance_embedder is not None:
-            g = guidance.to(self.dtype) * 1000
-            emb = emb + _mlp(timestep_projection(g, s.timestep_dim).to(self.dtype), self.guidance_embedder)
-        return emb + _mlp(pooled.to(self.dtype), self.text_embedder)
+            scalars.append(guidance.to(self.dtype))
+            mlps.append(self.guidance_embedder)
+        return embed(scalars, mlps, pooled.to(self.dtype), self.text_embedder, self.shape.timestep_dim,
+                     silu=silu)
 
     @torch.inference_mode()
     def forward(self, hidden_states, encoder_hidden_states, pooled_projections, timestep, img_ids,
@@ -423,8 +412,8 @@ class FluxTransformer:
                 hidden_states = index_select_rows(hidden_states, 1, layout.order)
                 img_ids = index_select_rows(img_ids.contiguous(), 0, layout.order)
         cos, sin = rotary_tables(torch.cat([txt_ids, img_ids]).to(self.device))
-        double_mods, single_mods, out_mods = self._modulations(F.silu(self.temb(timestep, guidance,
-                                                                                pooled_projections)))
+        double_mods, single_mods, out_mods = self._modulations(self.temb(timestep, guidance,
+                                                                         pooled_projections, silu=True))
         x = F.linear(hidden_states.to(self.dtype), *self.x_embedder)
         c = F.linear(encoder_hidden_states.to(self.dtype), *self.context_embedder)
         (sx, scx, *_), (sc, scc, *_) = double_mods[0]

@@ -158,6 +158,27 @@ int hb_qk_prep(const void* src_text, const void* src_image, int64_t text_batch_s
 int hb_rotary_tables(const float* ids, int64_t tokens, double theta, const int32_t* axes_dim,
                      float* cos, float* sin, hb_stream_t stream);
 
+/* Linear layers of 1..8 rows in one launch (the conditioning layers of the transformer reference
+ * hilberta/flux_adapter.py wraps: diffusers 0.36.0 CombinedTimestepGuidanceTextProjEmbeddings and
+ * the AdaLN modulation projections).  Output o (of `outputs`) is the sum of `sum` (1..3) layers
+ * i = o*sum .. o*sum + sum - 1:
+ *   out[o][b, c] = act(sum_i round(x[i][b, :] . weights[i][c, :] + biases[i][c])),  act = SiLU or none
+ * with fp32 products and sums; each layer's value, each addition and the SiLU are rounded to the
+ * 16-bit type.  All arrays are host arrays of outputs*sum entries (out and n: outputs entries) and
+ * hold at most 64 layers; x[i] is [batch, k[i]] with x_strides[i] elements between rows, weights[i]
+ * [n[o], k[i]] contiguous, biases[i] [n[o]] or NULL, out[o] [batch, n[o]] contiguous.  k a multiple
+ * of 8; x and weights 16-byte aligned. */
+int hb_linear_rows(int32_t outputs, int32_t sum, int32_t batch, int32_t dtype, int32_t silu,
+                   const void* const* x, const int64_t* x_strides, const void* const* weights,
+                   const void* const* biases, void* const* out, const int32_t* n, const int32_t* k,
+                   hb_stream_t stream);
+
+/* Sinusoidal embeddings of one or two sets of `batch` scalars (16-bit, t1 may be NULL): row
+ * s*batch + b of out is [cos | sin] (dim / 2 each) of round(1000 t_s[b]) * 10000^(-j / (dim / 2)), in
+ * fp32, rounded.  Diffusers 0.36.0 get_timestep_embedding as the FLUX embedders call it. */
+int hb_sinusoid_rows(const void* t0, const void* t1, int32_t batch, int32_t dim, int32_t dtype,
+                     void* out, hb_stream_t stream);
+
 /* Gated residual update + AdaLN modulation, one pass per row (FLUX blocks).  For each of
  * batch x rows rows of `hidden` values (row i of batch b at base + b*batch_stride + i*row_stride):
  *   r = x + gate[b] * y            (skipped when y is NULL: r = x)
