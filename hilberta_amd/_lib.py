@@ -60,6 +60,7 @@ SIGNATURES = {
         _c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _p, _p, _p, _p, _p, _p, _p, _p],
     ),
     "hb_sinusoid_rows": (_c_int, [_p, _p, _c_int, _c_int, _c_int, _p, _p]),
+    "hb_euler_step": (_c_int, [_p, _p, _c_f32, _p, _c_i64, _c_int, _p]),
     "hb_adaln_modulate": (
         _c_int,
         [_c_int, _c_int, _c_int, _c_int, _c_f32, _p, _c_i64, _c_i64, _p, _c_i64, _c_i64, _p, _c_i64,

@@ -25,7 +25,10 @@ import math
 import numpy as np
 import torch
 
+from . import _lib
 from .layout import index_select_rows
+
+_DTYPES = {torch.bfloat16: 0, torch.float16: 1}
 
 # FLUX.1-dev scheduler configuration (scheduler_config.json of the model repository)
 BASE_IMAGE_SEQ_LEN = 256
@@ -56,6 +59,22 @@ def flux_sigmas(steps, image_seq_len):
     return torch.cat([sigmas, torch.zeros(1)]), timesteps
 
 
+def euler_step(latents, pred, step):
+    """pred's type of (float32(latents) + step * float32(pred)): one pass (csrc/euler.hip) for plain
+    contiguous 16-bit device tensors, the torch sequence otherwise."""
+    if (latents.dtype in _DTYPES and latents.dtype == pred.dtype and latents.shape == pred.shape
+            and _lib.is_plain(latents, pred) and latents.device == pred.device
+            and latents.is_contiguous() and pred.is_contiguous()
+            and not (latents.data_ptr() | pred.data_ptr()) % 16):
+        out = torch.empty_like(pred)
+        with torch.cuda.device(pred.device):
+            rc = _lib.load().hb_euler_step(latents.data_ptr(), pred.data_ptr(), step, out.data_ptr(),
+                                           pred.numel(), _DTYPES[pred.dtype], _lib.stream_ptr(pred.device))
+        _lib.check(rc, "hb_euler_step")
+        return out
+    return (latents.float() + step * pred.float()).to(pred.dtype)
+
+
 @torch.inference_mode()
 def sample_flux(model, latents, encoder_hidden_states, pooled_projections, img_ids, txt_ids, *,
                 steps, guidance=3.5, attention=None, layout_scope="sampling"):
@@ -83,14 +102,15 @@ def sample_flux(model, latents, encoder_hidden_states, pooled_projections, img_i
         info["sampling_layout_read_write_bytes"] += 2 * (latents.numel() * latents.element_size()
                                                          + img_ids.numel() * img_ids.element_size())
     guidance_t = torch.full((B,), guidance, device=latents.device, dtype=torch.float32)
+    timesteps = timesteps.to(latents.device)   # one copy: a copy per step would drain the stream
     for i in range(steps):
-        t = timesteps[i].expand(B).to(latents.device)
+        t = timesteps[i].expand(B)
         pred = model(latents, encoder_hidden_states, pooled_projections,
                      t.to(latents.dtype) / NUM_TRAIN_TIMESTEPS, img_ids, txt_ids, guidance_t,
                      attention=attention, layout_scope=layout_scope)
         info["transformer_calls"] += 1
         step = float(sigmas[i + 1] - sigmas[i])
-        latents = (latents.float() + step * pred.float()).to(pred.dtype)
+        latents = euler_step(latents, pred, step)
     if packed:
         latents = index_select_rows(latents, 1, layout.inverse)
         info["sampling_inverse_calls"] += 1

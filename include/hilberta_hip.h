@@ -179,6 +179,12 @@ int hb_linear_rows(int32_t outputs, int32_t sum, int32_t batch, int32_t dtype, i
 int hb_sinusoid_rows(const void* t0, const void* t1, int32_t batch, int32_t dim, int32_t dtype,
                      void* out, hb_stream_t stream);
 
+/* Flow-matching Euler update of n 16-bit values: out = round(x + step * y) in fp32, the product
+ * rounded before the sum (diffusers 0.36.0 FlowMatchEulerDiscreteScheduler.step, in the sampling loop
+ * of reference hilberta/sampling_layout.py:20-148).  16-byte aligned; out may be x or y. */
+int hb_euler_step(const void* x, const void* y, float step, void* out, int64_t n, int32_t dtype,
+                  hb_stream_t stream);
+
 /* Gated residual update + AdaLN modulation, one pass per row (FLUX blocks).  For each of
  * batch x rows rows of `hidden` values (row i of batch b at base + b*batch_stride + i*row_stride):
  *   r = x + gate[b] * y            (skipped when y is NULL: r = x)
