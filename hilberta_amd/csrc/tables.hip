@@ -632,9 +632,10 @@ extern "C" int hb_quad_rows(const int32_t* kv_indices, const int32_t* kv_flags,
 // The global-prefix length (the shared blocks of the layout) stays on the device: the phase
 // kernels read it from status[0], so nothing synchronises before the table widths are known.
 //
-//   P1 composite order (grid-wide) + clearing the four phases' score matrices
-//   P2 one workgroup: block packing, image order and its inverse, the permutation check, status
-//   P3 bridge scores of all four phases (atomic adds per raster 4-neighbour pair) + base rows
+//   P1 composite order (grid-wide), shared tokens per block + clearing the score matrices, status
+//   P2 block packing, image order and its inverse (a wave per block), shared blocks -> status[0]
+//   P3 permutation check, bridge scores of all four phases (atomic adds per raster 4-neighbour
+//      pair) + base rows
 //   P4 top-K per (phase, query block), reciprocal bridge bits
 //   P5 paired row counts per phase -> status[3 + phase] = widest row
 //   -- host reads status (n_shared, partial, bad order, four widths), allocates exact tables --
@@ -646,108 +647,84 @@ namespace {
 
 constexpr int PLAN_PHASES = 4;
 
-__global__ void plan_composite_kernel(int g, int64_t* original, int64_t* inverse, int32_t* scores,
-                                      int64_t score_words) {
+// One wave per 64-token block of the composite order (its tokens are its lanes), then the score
+// words.  block_shared[b] counts the block's tokens inside the shared square.
+__global__ void plan_composite_kernel(int g, int shared, int64_t* original, int64_t* inverse,
+                                      int32_t* block_shared, int32_t* scores, int64_t score_words,
+                                      int32_t* status) {
   const int64_t n = (int64_t)g * g;
   const int64_t total = n > score_words ? n : score_words;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-    if (i < n) {
+  const int start = 3 * g / 8, end = 5 * g / 8;
+  const int64_t first = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (first >= 1 && first < 3 + PLAN_PHASES) status[first] = 0;
+  for (int64_t i = first; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+    if (i < n) {  // n is a multiple of 64: whole waves
       const int64_t half = n / 2;
       const int64_t src = n / 4 + (i < half ? i : i - half);
       const int64_t h = hilbert_raster(src, g);
       const int64_t tok = i < half ? h : n - 1 - h;
       original[i] = tok;
       inverse[tok] = i;
+      const int y = (int)(tok / g), x = (int)(tok % g);
+      const bool in = shared && y >= start && y < end && x >= start && x < end;
+      const int cnt = __popcll(__ballot(in));
+      if ((threadIdx.x & 63) == 0) block_shared[i >> 6] = cnt;
     }
     if (i < score_words) scores[i] = 0;
   }
 }
 
-// The block packing of pack_blocks_kernel, then (same workgroup, after a barrier) the image order,
-// its inverse and the permutation check of image_order_kernel / order_check_kernel.
-__global__ void __launch_bounds__(1024) plan_pack_kernel(int g, int bs, int shared,
-                                                         const int64_t* original, int text_blocks,
-                                                         int64_t* packed, int64_t* to_physical,
-                                                         int64_t* order, int64_t* inverse_order,
-                                                         int32_t* status) {
-  const int64_t n = (int64_t)g * g;
-  const int nb = (int)(n / bs);
-  __shared__ int s_total[3];
-  __shared__ int s_scan[1024];
-  const int t = threadIdx.x;
-  const int per = (nb + 1023) / 1024;
-  const int lo = min(t * per, nb), hi = min(lo + per, nb);
-  const int start = 3 * g / 8, end = 5 * g / 8;
-  auto shared_tokens = [&](int b) {
-    int cnt = 0;
-    if (shared) {
-      for (int j = 0; j < bs; ++j) {
-        const int64_t tok = original[(int64_t)b * bs + j];
-        const int y = (int)(tok / g), x = (int)(tok % g);
-        cnt += (y >= start && y < end && x >= start && x < end);
-      }
-    }
-    return cnt;
-  };
-  int my_shared = 0, partial = 0;
-  for (int b = lo; b < hi; ++b) {
-    const int cnt = shared_tokens(b);
-    if (cnt != 0 && cnt != bs) partial = 1;
-    my_shared += (cnt == bs);
+// Block packing (shared blocks first, each group in composite order) and the image order, one wave
+// per block: every wave counts the whole list's shared blocks before its own (nb / 64 loads per lane,
+// served by L2), so no workgroup waits for another.  As one workgroup's scan and walk over the
+// image this took 23 us at 2048 px and was the largest launch of a plan.
+__global__ void plan_pack_kernel(int nb, int text_blocks, const int64_t* original,
+                                 const int32_t* block_shared, int64_t* packed,
+                                 int64_t* to_physical, int64_t* order, int64_t* inverse_order,
+                                 int32_t* status) {
+  const int b = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  const int lane = threadIdx.x & 63;
+  if (b >= nb) return;
+  const int64_t tok = original[(int64_t)b * 64 + lane];
+  int before = 0, n_shared = 0;
+  for (int i = lane; i < nb; i += 64) {
+    const int full = block_shared[i] == 64;
+    n_shared += full;
+    before += full && i < b;
   }
-  s_scan[t] = my_shared;
-  if (t == 0) {
-    s_total[1] = 0;
-    s_total[2] = 0;
+  for (int off = 32; off >= 1; off >>= 1) {
+    before += __shfl_xor(before, off);
+    n_shared += __shfl_xor(n_shared, off);
   }
-  __syncthreads();
-  if (partial) atomicOr(&s_total[1], 1);
-  for (int off = 1; off < 1024; off *= 2) {
-    const int v = t >= off ? s_scan[t - off] : 0;
-    __syncthreads();
-    s_scan[t] += v;
-    __syncthreads();
-  }
-  const int n_shared = s_scan[1023];
-  int sh_before = s_scan[t] - my_shared;
-  int ord_before = lo - sh_before;
-  for (int b = lo; b < hi; ++b) {
-    const int slot = shared_tokens(b) == bs ? sh_before++ : n_shared + ord_before++;
+  const int own = block_shared[b];
+  const int slot = own == 64 ? before : n_shared + b - before;
+  const int64_t i = (int64_t)slot * 64 + lane;
+  order[i] = tok;
+  if (tok >= 0 && tok < (int64_t)nb * 64) inverse_order[tok] = i;
+  if (lane == 0) {
     packed[slot] = b;
     to_physical[b] = slot + text_blocks;
+    if (own != 0 && own != 64) atomicOr(&status[1], 1);
+    if (b == 0) status[0] = n_shared;
   }
-  __syncthreads();  // packed complete (global writes of this workgroup are visible after it)
-  for (int64_t i = t; i < n; i += 1024) {
-    const int64_t tok = original[packed[i / bs] * bs + i % bs];
-    order[i] = tok;
-    if (tok >= 0 && tok < n) inverse_order[tok] = i;
-  }
-  __syncthreads();
-  int bad = 0;
-  for (int64_t i = t; i < n; i += 1024) {
-    const int64_t tok = order[i];
-    bad |= tok < 0 || tok >= n || inverse_order[tok] != i;
-  }
-  if (bad) atomicOr(&s_total[2], 1);
-  __syncthreads();
-  if (t == 0) {
-    status[0] = n_shared;
-    status[1] = s_total[1];
-    status[2] = s_total[2];
-  }
-  if (t < PLAN_PHASES) status[3 + t] = 0;
 }
 
 // Bridge scores of the four phases (blocks [0, score_blocks)) and their base rows (the rest).
 __global__ void plan_scores_base_kernel(int g, int bs, int tiles, int text_blocks, int score_blocks,
                                         const int64_t* inverse, const int64_t* packed,
-                                        const int32_t* status, int32_t* scores, uint32_t* bits) {
+                                        const int64_t* order, const int64_t* inverse_order,
+                                        int32_t* status, int32_t* scores, uint32_t* bits) {
   const int64_t n = (int64_t)g * g;
   const int nb = (int)(n / bs);
   const int T = text_blocks + nb;
   const int words = (T + 31) / 32;
   const int64_t width = n / tiles;
   if ((int)blockIdx.x < score_blocks) {
+    // the image order of the launch before must be a permutation of the image tokens
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)score_blocks * blockDim.x) {
+      const int64_t tok = order[i];
+      if (tok < 0 || tok >= n || inverse_order[tok] != i) atomicOr(&status[2], 1);
+    }
     const int64_t pairs = 2 * (int64_t)g * (g - 1);
     for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < pairs; p += (int64_t)score_blocks * blockDim.x) {
       int64_t a, c;
@@ -821,18 +798,29 @@ __global__ void plan_topk_bits_kernel(int g, int bs, int tiles, int k, int text_
   const int gb = text_blocks + status[0];
   uint32_t* pb = bits + (int64_t)ph * nb * words;
   const int pq = (int)to_physical[q];
-  uint64_t bound = ~0ull;
-  for (int j = 0; j < k; ++j) {
-    uint64_t best = 0;
-    for (int key = lane; key < nb; key += 64) {
-      const int s = sc[key];
-      if (s <= 0) continue;
-      const int rolled = ((key - offset_blocks) % nb + nb) % nb;
-      const uint64_t code = ((uint64_t)(uint32_t)s << 32) | (uint32_t)(nb - 1 - rolled);
-      if (code < bound && code > best) best = code;
+  // each lane's four best codes in one pass over the row (k passes waited k times for the loads)
+  uint64_t top[4] = {0, 0, 0, 0};
+#pragma unroll 4
+  for (int key = lane; key < nb; key += 64) {
+    const int s = sc[key];
+    const int rolled = key >= offset_blocks ? key - offset_blocks : key - offset_blocks + nb;
+    uint64_t code = s > 0 ? ((uint64_t)(uint32_t)s << 32) | (uint32_t)(nb - 1 - rolled) : 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint64_t hi = code > top[i] ? code : top[i];
+      code = code > top[i] ? top[i] : code;
+      top[i] = hi;
     }
-    best = wave_max_u64(best);
+  }
+  for (int j = 0; j < k; ++j) {
+    const uint64_t best = wave_max_u64(top[0]);
     if (!best) break;
+    if (top[0] == best) {  // codes are unique: one lane gives its best up
+      top[0] = top[1];
+      top[1] = top[2];
+      top[2] = top[3];
+      top[3] = 0;
+    }
     if (lane == 0) {
       const int rolled = nb - 1 - (int)(best & 0xffffffffu);
       const int key = (rolled + offset_blocks) % nb;
@@ -840,28 +828,38 @@ __global__ void plan_topk_bits_kernel(int g, int bs, int tiles, int k, int text_
       if (pq >= gb) atomicOr(&pb[(int64_t)(pq - gb) * words + pk / 32], 1u << (pk % 32));
       if (pk >= gb) atomicOr(&pb[(int64_t)(pk - gb) * words + pq / 32], 1u << (pq % 32));
     }
-    bound = best;
   }
 }
 
 // Paired counts of the four phases: one wave per (phase, paired row); the widest row of each
-// phase goes to status[3 + phase].
-__global__ void plan_counts_kernel(int nb, int words, int T, int text_blocks, int ratio,
-                                   const uint32_t* bits, int32_t* status) {
-  const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+// phase goes to status[3 + phase].  A workgroup's sixteen rows meet in LDS first: with every row's
+// wave on the same four words the launch took 8.5 us at 2048 px, 3.5 us so.
+constexpr int COUNT_TPB = 1024;
+
+__global__ __launch_bounds__(COUNT_TPB) void plan_counts_kernel(int nb, int words, int T,
+                                                                int text_blocks, int ratio,
+                                                                const uint32_t* bits,
+                                                                int32_t* status) {
+  __shared__ int s_max[PLAN_PHASES];
+  if (threadIdx.x < PLAN_PHASES) s_max[threadIdx.x] = 0;
+  __syncthreads();
+  const int wave = (blockIdx.x * COUNT_TPB + threadIdx.x) >> 6;
   const int lane = threadIdx.x & 63;
   const int prows_max = nb / 2;
-  if (wave >= PLAN_PHASES * prows_max) return;
   const int ph = wave / prows_max, pr = wave - ph * prows_max;
   const int nq = T - text_blocks - status[0];
-  if (pr >= nq / 2) return;  // (an odd nq is rejected on the host)
-  const uint32_t* ra = bits + ((int64_t)ph * nb + 2 * pr) * words;
-  const uint32_t* rb = ra + words;
-  const int kblocks = (T + ratio - 1) / ratio;
-  int c = 0;
-  for (int kb = lane; kb < kblocks; kb += 64) c += pair_flag(ra, rb, kb, ratio) != 0;
-  for (int off = 32; off >= 1; off >>= 1) c += __shfl_xor(c, off);
-  if (lane == 0) atomicMax(&status[3 + ph], c);
+  if (ph < PLAN_PHASES && pr < nq / 2) {  // (an odd nq is rejected on the host)
+    const uint32_t* ra = bits + ((int64_t)ph * nb + 2 * pr) * words;
+    const uint32_t* rb = ra + words;
+    const int kblocks = (T + ratio - 1) / ratio;
+    int c = 0;
+    for (int kb = lane; kb < kblocks; kb += 64) c += pair_flag(ra, rb, kb, ratio) != 0;
+    for (int off = 32; off >= 1; off >>= 1) c += __shfl_xor(c, off);
+    if (lane == 0) atomicMax(&s_max[ph], c);
+  }
+  __syncthreads();
+  if (threadIdx.x < PLAN_PHASES && s_max[threadIdx.x])
+    atomicMax(&status[3 + threadIdx.x], s_max[threadIdx.x]);
 }
 
 struct PlanOut {
@@ -937,24 +935,29 @@ extern "C" int hb_paired_plan_tables(int32_t grid_size, int32_t tile_count, int3
   int32_t* scores = (int32_t*)scratch;
   uint32_t* bits = (uint32_t*)(scores + (int64_t)PLAN_PHASES * nb * nb);
   const int64_t score_words = (int64_t)PLAN_PHASES * nb * nb;
+  // the per-block shared counts live in the bitmaps' space until the base rows are written
+  int32_t* block_shared = (int32_t*)bits;
   hipLaunchKernelGGL(plan_composite_kernel, dim3(grid_for(n > score_words ? n : score_words)),
-                     dim3(TPB), 0, stream, grid_size, original_order, inverse_original, scores,
-                     score_words);
-  hipLaunchKernelGGL(plan_pack_kernel, dim3(1), dim3(1024), 0, stream, grid_size, bs, shared,
-                     (const int64_t*)original_order, text_blocks, physical_original_blocks,
-                     original_to_physical, image_order, inverse_image_order, status);
+                     dim3(TPB), 0, stream, grid_size, shared, original_order, inverse_original,
+                     block_shared, scores, score_words, status);
+  hipLaunchKernelGGL(plan_pack_kernel, dim3((nb + TPB / 64 - 1) / (TPB / 64)), dim3(TPB), 0, stream,
+                     nb, text_blocks, (const int64_t*)original_order, (const int32_t*)block_shared,
+                     physical_original_blocks, original_to_physical, image_order,
+                     inverse_image_order, status);
   const int score_blocks = grid_for(2 * n);
   const int base_blocks = grid_for((int64_t)PLAN_PHASES * nb * ((T + 63) / 64) * 64);
   hipLaunchKernelGGL(plan_scores_base_kernel, dim3(score_blocks + base_blocks), dim3(TPB), 0,
                      stream, grid_size, bs, tile_count, text_blocks, score_blocks,
                      (const int64_t*)inverse_original, (const int64_t*)physical_original_blocks,
-                     (const int32_t*)status, scores, bits);
+                     (const int64_t*)image_order, (const int64_t*)inverse_image_order, status,
+                     scores, bits);
   hipLaunchKernelGGL(plan_topk_bits_kernel, dim3(((int64_t)PLAN_PHASES * nb * 64 + TPB - 1) / TPB),
                      dim3(TPB), 0, stream, grid_size, bs, tile_count, k, text_blocks,
                      (const int32_t*)scores, (const int64_t*)original_to_physical,
                      (const int32_t*)status, bits);
-  hipLaunchKernelGGL(plan_counts_kernel, dim3(((int64_t)PLAN_PHASES * (nb / 2) * 64 + TPB - 1) / TPB),
-                     dim3(TPB), 0, stream, nb, words, T, text_blocks, key_block_size / 64,
+  hipLaunchKernelGGL(plan_counts_kernel,
+                     dim3(((int64_t)PLAN_PHASES * (nb / 2) * 64 + COUNT_TPB - 1) / COUNT_TPB),
+                     dim3(COUNT_TPB), 0, stream, nb, words, T, text_blocks, key_block_size / 64,
                      (const uint32_t*)bits, status);
   HB_HIP(hipGetLastError());
   return HB_OK;
