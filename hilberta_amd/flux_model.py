@@ -200,25 +200,46 @@ def _gelu_linear(x, weight, bias):
     return torch._addmm_activation(bias, flat, weight.t(), use_gelu=True).view(*x.shape[:-1], -1)
 
 
-def _joint_ranges(T, N):
-    """Row ranges [text | image] of a joint sequence of T text and N - T image tokens.
-
-    The single blocks' GEMMs run once per range: hipBLASLt takes a joint 16896-row GEMM at
-    1.05-1.2 PFLOP/s but the 16384 image rows alone at 1.5-1.8 (measured on MI355X: 12288 x 3072
-    weights 1.060 -> 0.846 ms with the 512 text rows as a second GEMM, 20-26 % less for each of
-    the four shapes of a single block)."""
-    return ((0, T), (T, N))
+_TILE, _CUS = 256, 256
 
 
-def _linear_rows(x, weight, bias, out, T, *, gelu=False):
-    """out = x @ weight^T + bias (GELU(tanh) in the epilogue if ``gelu``), one GEMM per batch
-    element and joint-sequence range, written in place into ``out``."""
-    for b in range(x.shape[0]):
-        for lo, hi in _joint_ranges(T, x.shape[1]):
-            if gelu:
-                torch._addmm_activation(bias, x[b, lo:hi], weight.t(), use_gelu=True, out=out[b, lo:hi])
-            else:
-                torch.addmm(bias, x[b, lo:hi], weight.t(), out=out[b, lo:hi])
+def _gemm_rounds(rows, columns):
+    """Rounds of 256 x 256 output tiles a [rows, columns] GEMM takes on the 256 compute units."""
+    return -(-(-(-rows // _TILE) * -(-columns // _TILE)) // _CUS)
+
+
+def _row_parts(T, shape, columns):
+    """How a single block's GEMM of ``columns`` outputs walks joint rows [B, N] of T text and N - T
+    image tokens: None for all rows at once, else the (batch, first, end) of each GEMM.
+
+    The text rows are a GEMM of their own unless the joint rows fill fewer rounds of tiles, which
+    decides every shape measured on MI355X (3072-wide model, 512 text rows, joint / split us): with
+    16384 image rows a tie, and the image rows alone fill whole rounds (9216 columns 735 / 659, 12288
+    1037 / 942, 3072 313 / 233, 3072 of depth 12288 1088 / 891); with 4096 the joint rows win where
+    they save the text's round (195 / 225, 66 / 85, 242 / 290) and lose on a tie (12288: 282 / 272);
+    with 1024 likewise (82 / 99, 36 / 47, 116 / 149; 126 / 115)."""
+    B, N = shape
+    split = B * (_gemm_rounds(T, columns) + _gemm_rounds(N - T, columns))
+    if _gemm_rounds(B * N, columns) < split:
+        return None
+    return [(b, lo, hi) for b in range(B) for lo, hi in ((0, T), (T, N))]
+
+
+def _linear_rows(x, weight, bias, out, T, *, gelu=False, add=None):
+    """out = x @ weight^T + bias (GELU(tanh) in the epilogue if ``gelu``; plus the bias-free product
+    of ``add`` = (x, weight)) over contiguous joint rows [B, N, K], written into ``out`` by the GEMMs
+    of _row_parts."""
+    parts = _row_parts(T, x.shape[:2], out.shape[-1])
+    rows = ((lambda t: [t.view(-1, t.shape[-1])]) if parts is None
+            else (lambda t: [t[b, lo:hi] for b, lo, hi in parts]))
+    more = rows(add[0]) if add else ()
+    for i, (xr, outr) in enumerate(zip(rows(x), rows(out))):
+        if gelu:
+            torch._addmm_activation(bias, xr, weight.t(), use_gelu=True, out=outr)
+        else:
+            torch.addmm(bias, xr, weight.t(), out=outr)
+        if add:
+            outr.addmm_(more[i], add[1].t())
 
 
 class FluxTransformer:
@@ -362,11 +383,7 @@ class FluxTransformer:
         (wa, ba), (wm, _) = w["out_attn"], w["out_mlp"]
         o = o.view(B, N, C)
         p = h.new_empty(B, N, C)                                           # proj_out([attn | mlp])
-        for b in range(B):
-            for lo, hi in _joint_ranges(T, N):
-                pr = p[b, lo:hi]
-                torch.addmm(ba, o[b, lo:hi], wa.t(), out=pr)
-                pr.addmm_(mlp[b, lo:hi], wm.t())
+        _linear_rows(o, wa, ba, p, T, add=(mlp, wm))
         del o, mlp
         shift, scale = next_mods
         if layer < self.shape.blocks - 1:
