@@ -13,8 +13,9 @@ rebuilt on hand-written HIP kernels behind a C ABI (include/hilberta_hip.h):
                     gated-residual AdaLN pass, one HIP kernel each
   flux_model / sampling_layout
                     a FLUX-shaped denoiser step on these kernels and the sampling-scope layout
-  ops               the entry points as torch custom ops (torch.ops.hilberta_hip.*), with fake
-                    implementations for tracing
+  flux_cond         conditioning layers of a few rows (embedders, modulations), streamed by HIP
+  ops               the entry points as native torch operators (torch.ops.hilberta_hip.*), with
+                    fake implementations for tracing
 
 The modules keep the reference package's call surface.  There is no CPU fallback: the HIP library
 (python -m hilberta_amd.build) and a GPU are required for every computation.

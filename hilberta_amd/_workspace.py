@@ -1,4 +1,4 @@
-"""Per-(device, stream) workspaces for the attention kernels.
+"""Per-(device, stream) workspaces for the attention kernels (csrc/torch_ops.cpp holds them).
 
 A workspace holds the persistent kernel's work-queue counters (zero-filled once at allocation;
 every launch leaves them at zero) and the partial results of split global query tiles.  Keying
@@ -15,9 +15,18 @@ from __future__ import annotations
 
 import torch
 
-from . import _lib
+from . import _lib, ops
 
-_CACHE: dict = {}
+
+class _Cache:
+    """The (device, stream) keys of the cached eager workspaces."""
+
+    def __iter__(self):
+        keys = ops.workspace_keys()
+        return iter(list(zip(keys[::2], keys[1::2])))
+
+
+_CACHE = _Cache()
 
 
 def attention_workspace(device, batch, heads, tokens, head_dim, global_tokens, width,
@@ -27,17 +36,9 @@ def attention_workspace(device, batch, heads, tokens, head_dim, global_tokens, w
         int(all_queries))
     if need < 0:
         _lib.check(1, "hb_attention_workspace_bytes")
-    if torch.cuda.is_current_stream_capturing():
-        return torch.zeros(max(need, 1 << 16), dtype=torch.uint8, device=device)
-    stream = torch.cuda.current_stream(device)
-    key = (str(device), stream.cuda_stream)
-    ws = _CACHE.get(key)
-    if ws is None or ws.numel() < need:
-        ws = torch.zeros(max(need, 1 << 16), dtype=torch.uint8, device=device)
-        _CACHE[key] = ws
-    return ws
+    return ops.attention_workspace(torch.device(device), need)
 
 
 def clear() -> None:
     """Drop the cached eager workspaces."""
-    _CACHE.clear()
+    ops.clear_workspaces()

@@ -1,9 +1,9 @@
-"""Build libhilberta_hip.so (gfx950) in-tree with hipcc.
+"""Build libhilberta_hip.so (gfx950, hipcc) and libhilberta_torch.so (the torch operators) in-tree.
 
-    python -m hilberta_amd.build          # compile every csrc/*.hip, link the shared library
+    python -m hilberta_amd.build          # compile every csrc/*.hip and torch_ops.cpp, link both
 
-Objects go to hilberta_amd/_build/, the library to hilberta_amd/libhilberta_hip.so; both are
-git-ignored and travel with the source tree to the GPU box.
+Objects go to hilberta_amd/_build/, the libraries to hilberta_amd/; all are git-ignored.
+libhilberta_torch.so is host code over the C ABI, built against the installed torch.
 """
 
 from __future__ import annotations
@@ -19,6 +19,8 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 OUT = PKG / "_build"
 LIB = PKG / "libhilberta_hip.so"
+TORCH_LIB = PKG / "libhilberta_torch.so"
+TORCH_SRC = CSRC / "torch_ops.cpp"
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [
@@ -62,11 +64,49 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def _host_compiler() -> str:
+    for cand in (os.environ.get("CXX"), shutil.which("g++"), shutil.which("c++")):
+        if cand and shutil.which(cand):
+            return cand
+    raise RuntimeError("a host C++ compiler (g++) is required to build the torch operators")
+
+
+def _run(cmd, what):
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode:
+        raise RuntimeError(f"{what} failed:\n{proc.stderr}")
+
+
+def _compile_torch_ops() -> Path:
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    obj = OUT / (TORCH_SRC.stem + ".o")
+    includes = [arg for path in include_paths("cuda") for arg in ("-isystem", path)]
+    _run([_host_compiler(), "-O2", "-std=c++17", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes, "-c", str(TORCH_SRC),
+          "-o", str(obj)], f"compiling {TORCH_SRC.name}")
+    return obj
+
+
+def _link_torch_ops(obj: Path) -> None:
+    """Against the library beside it ($ORIGIN) and the installed torch, which is loaded before it."""
+    from torch.utils.cpp_extension import library_paths
+
+    tmp = TORCH_LIB.with_suffix(".so.tmp")
+    _run([_host_compiler(), "-shared", str(obj), "-o", str(tmp), f"-L{PKG}", f"-l:{LIB.name}", "-Wl,-rpath,$ORIGIN",
+          *(f"-L{path}" for path in library_paths("cuda")), "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip"],
+         f"linking {TORCH_LIB.name}")
+    os.replace(tmp, TORCH_LIB)
+
+
 def build(verbose: bool = True) -> Path:
     OUT.mkdir(exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))
     with cf.ThreadPoolExecutor(max_workers=min(8, len(sources))) as pool:
+        torch_ops = pool.submit(_compile_torch_ops)
         objects = list(pool.map(_compile, sources))
+        torch_object = torch_ops.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
@@ -79,8 +119,9 @@ def build(verbose: bool = True) -> Path:
     if stubs:
         raise RuntimeError(f"link left {len(stubs)} kernel launch stubs undefined, e.g. {stubs[0]}")
     os.replace(tmp, LIB)
+    _link_torch_ops(torch_object)
     if verbose:
-        print(f"built {LIB} from {len(sources)} sources")
+        print(f"built {LIB} from {len(sources)} sources, and {TORCH_LIB.name}")
     return LIB
 
 

@@ -49,53 +49,59 @@ def paired_attention(
     tuning keywords are validated as in the reference but select no code path.  ``lse`` may be a
     contiguous float32 [B,H,N] tensor that receives the natural-log row logsumexp.
     """
-    if q.ndim != 4 or k.shape != q.shape or v.shape != q.shape or any(x <= 0 for x in q.shape):
+    # (sizes, strides and dtypes are read once: each read of a tensor attribute costs the host about as
+    # much as a comparison, and a short call is as long as its checks)
+    shape, dtype, device = q.shape, q.dtype, q.device
+    if q.ndim != 4 or k.shape != shape or v.shape != shape or min(shape) <= 0:
         raise ValueError("Equal nonempty B,H,N,D Q/K/V required")
-    if q.shape[-1] not in (64, 128) or any(x.stride(-1) != 1 for x in (q, k, v)):
+    strides = q.stride(), k.stride(), v.stride()
+    if shape[-1] not in (64, 128) or any([s[-1] != 1 for s in strides]):
         raise ValueError("D64 or128 must be contiguous")
-    if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype:
+    if dtype not in (torch.float16, torch.bfloat16) or k.dtype != dtype or v.dtype != dtype:
         raise TypeError("Q/K/V must share BF16/FP16 dtype")
-    if not q.is_cuda or k.device != q.device or v.device != q.device:
+    if not q.is_cuda or k.device != device or v.device != device:
         raise ValueError("Q/K/V must be on the same CUDA device")
-    if any(any(s <= 0 for s in x.stride()[:3]) for x in (q, k, v)):
+    if any([min(s[:3]) <= 0 for s in strides]):
         raise ValueError("Positive Q/K/V outer strides required")
-    if torch.is_grad_enabled() and any(x.requires_grad for x in (q, k, v)):
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
         raise ValueError("Inference only; disable autograd")
-    for name in ("tokens", "global_tokens", "key_block_size"):
-        value = getattr(metadata, name)
-        if isinstance(value, bool) or not isinstance(value, Integral):
+    N, G, key_block = metadata.tokens, metadata.global_tokens, metadata.key_block_size
+    for value in (N, G, key_block):
+        if type(value) is not int and (isinstance(value, bool) or not isinstance(value, Integral)):
             raise TypeError("Integer metadata shape fields required")
-    N, G = metadata.tokens, metadata.global_tokens
-    if q.shape[-2] != N or G % 128 or N % 128 or not 0 <= G < N or metadata.key_block_size not in (64, 128):
+    if shape[-2] != N or G % 128 or N % 128 or not 0 <= G < N or key_block not in (64, 128):
         raise ValueError("Metadata/token shape mismatch or invalid128-token alignment")
     rows = (N - G) // 128
-    if metadata.kv_indices.ndim != 2 or metadata.kv_indices.shape[0] != rows or metadata.kv_indices.shape[1] < 1:
+    ids, flags, counts = metadata.kv_indices, metadata.kv_flags, metadata.kv_counts
+    table = ids.shape
+    if ids.ndim != 2 or table[0] != rows or table[1] < 1:
         raise ValueError("Paired index shape must match ordinary query pairs")
-    if metadata.kv_flags.shape != metadata.kv_indices.shape or metadata.kv_counts.shape != (rows,):
+    if flags.shape != table or counts.shape != (rows,):
         raise ValueError("Paired flag/count shape mismatch")
-    for x in (metadata.kv_indices, metadata.kv_flags, metadata.kv_counts):
-        if x.device != q.device or x.dtype != torch.int32 or not x.is_contiguous():
+    for x in (ids, flags, counts):
+        if x.device != device or x.dtype != torch.int32 or not x.is_contiguous():
             raise ValueError("Cached CUDA contiguous int32 metadata required")
     if global_strategy not in ("flash", "triton"):
         raise ValueError("Invalid global strategy")
-    if any(isinstance(x, bool) or not isinstance(x, Integral) for x in (num_warps, num_stages)):
+    if any([isinstance(x, bool) or not isinstance(x, Integral) for x in (num_warps, num_stages)]):
         raise TypeError("Integer launch tuning required")
     if num_warps not in (4, 8) or num_stages not in (1, 2, 3, 4):
         raise ValueError("Invalid launch tuning")
     if scale is not None and (isinstance(scale, bool) or not isinstance(scale, Real)):
         raise TypeError("scale must be a real scalar, never a tensor")
-    scale = q.shape[-1] ** -0.5 if scale is None else float(scale)
+    scale = shape[-1] ** -0.5 if scale is None else float(scale)
     if not math.isfinite(scale) or scale <= 0:
         raise ValueError("Positive finite scale required")
     if out is not None:
-        if out.shape != q.shape or out.dtype != q.dtype or out.device != q.device or out.stride(-1) != 1:
+        out_strides = out.stride()
+        if out.shape != shape or out.dtype != dtype or out.device != device or out_strides[-1] != 1:
             raise ValueError("Output must match Q shape/dtype/device with contiguous D")
-        if any(s <= 0 for s in out.stride()) or not _non_overlapping_strides(out):
+        if min(out_strides) <= 0 or not _non_overlapping_strides(out):
             raise ValueError("Positive non-overlapping output strides required")
         if torch.is_grad_enabled() and out.requires_grad:
             raise ValueError("Inference output cannot require gradients")
         begin, end = _tensor_byte_span(out)
-        for x in (q, k, v, metadata.kv_indices, metadata.kv_flags, metadata.kv_counts):
+        for x in (q, k, v, ids, flags, counts):
             first, last = _tensor_byte_span(x)
             if begin < last and first < end:
                 raise ValueError("Output cannot alias inputs or metadata")

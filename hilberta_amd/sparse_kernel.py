@@ -106,39 +106,42 @@ def explicit_mask(kv_indices, kv_counts, *, tokens, global_tokens=768, block_siz
 
 def _tensor_byte_span(tensor):
     """Conservative [begin, end) byte interval of a strided view (host metadata only)."""
-    begin = tensor.data_ptr()
-    extent = 1 + sum((size - 1) * stride for size, stride in zip(tensor.shape, tensor.stride()))
+    begin, extent = tensor.data_ptr(), 1
+    for size, stride in zip(tensor.shape, tensor.stride()):
+        extent += (size - 1) * stride
     return begin, begin + extent * tensor.element_size()
 
 
 def _non_overlapping_strides(tensor):
     extent = 1
-    for stride, size in sorted(
-        (stride, size) for stride, size in zip(tensor.stride(), tensor.shape) if size > 1
-    ):
-        if stride < extent:
-            return False
-        extent += (size - 1) * stride
+    for stride, size in sorted(zip(tensor.stride(), tensor.shape)):
+        if size > 1:
+            if stride < extent:
+                return False
+            extent += (size - 1) * stride
     return True
 
 
 def _check_inputs(q, k, v, kv_indices, kv_counts, global_tokens, block_size, out):
     """Host-side launch checks of reference sparse_kernel.py:188-250 (same messages)."""
-    if q.ndim != 4 or k.shape != q.shape or v.shape != q.shape or any(s <= 0 for s in q.shape):
+    # (sizes, strides and dtypes are read once: see paired_kernel.paired_attention)
+    shape, dtype, device = q.shape, q.dtype, q.device
+    if q.ndim != 4 or k.shape != shape or v.shape != shape or min(shape) <= 0:
         raise ValueError("Q/K/V must have equal, nonempty [B,H,N,D] shapes")
-    if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype:
+    if dtype not in (torch.float16, torch.bfloat16) or k.dtype != dtype or v.dtype != dtype:
         raise TypeError("Q/K/V must share FP16 or BF16 dtype")
-    if not q.is_cuda or k.device != q.device or v.device != q.device:
+    if not q.is_cuda or k.device != device or v.device != device:
         raise ValueError("Q/K/V must be on one CUDA device")
-    if torch.is_grad_enabled() and any(x.requires_grad for x in (q, k, v)):
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
         raise ValueError("sparse_attention is inference-only; disable autograd before calling")
-    if q.shape[-1] not in (64, 128) or any(x.stride(-1) != 1 for x in (q, k, v)):
+    strides = q.stride(), k.stride(), v.stride()
+    if shape[-1] not in (64, 128) or any([s[-1] != 1 for s in strides]):
         raise ValueError("D must be64 or128 and contiguous; outer strides may differ")
-    if any(any(stride <= 0 for stride in x.stride()[:3]) for x in (q, k, v)):
+    if any([min(s[:3]) <= 0 for s in strides]):
         raise ValueError("Q/K/V outer strides must be positive")
-    if any(isinstance(v_, bool) or not isinstance(v_, Integral) for v_ in (global_tokens, block_size)):
+    if any([isinstance(v_, bool) or not isinstance(v_, Integral) for v_ in (global_tokens, block_size)]):
         raise TypeError("global_tokens and block_size must be integers")
-    n = q.shape[-2]
+    n = shape[-2]
     if block_size != 64 or n % block_size or global_tokens % block_size or not 0 <= global_tokens < n:
         raise ValueError("N and global_tokens must align to64, with ordinary queries remaining")
     rows = (n - global_tokens) // block_size
@@ -149,17 +152,18 @@ def _check_inputs(q, k, v, kv_indices, kv_counts, global_tokens, block_size, out
         or kv_counts.shape != (rows,)
     ):
         raise ValueError("Metadata shape does not match the ordinary query partition")
-    if any(
-        x.device != q.device or x.dtype != torch.int32 or not x.is_contiguous()
+    if any([
+        x.device != device or x.dtype != torch.int32 or not x.is_contiguous()
         for x in (kv_indices, kv_counts)
-    ):
+    ]):
         raise ValueError("Metadata must be cached contiguous CUDA int32 tensors on the Q device")
     if out is not None:
-        if out.shape != q.shape or out.dtype != q.dtype or out.device != q.device or out.stride(-1) != 1:
+        out_strides = out.stride()
+        if out.shape != shape or out.dtype != dtype or out.device != device or out_strides[-1] != 1:
             raise ValueError(
                 "Provided output must match Q shape/dtype/device with contiguous last dimension"
             )
-        if any(stride <= 0 for stride in out.stride()) or not _non_overlapping_strides(out):
+        if min(out_strides) <= 0 or not _non_overlapping_strides(out):
             raise ValueError("Provided output must have positive, non-overlapping strides")
         if torch.is_grad_enabled() and out.requires_grad:
             raise ValueError("An inference output cannot require gradients")
@@ -173,7 +177,8 @@ def _check_inputs(q, k, v, kv_indices, kv_counts, global_tokens, block_size, out
 def _check_vector_layout(tensors):
     """The HIP kernel moves 16-byte vectors: base pointers 16-byte aligned, strides multiple of 8."""
     for x in tensors:
-        if x.data_ptr() % 16 or any(s % 8 for s in x.stride()[:3]):
+        s0, s1, s2 = x.stride()[:3]
+        if x.data_ptr() % 16 or (s0 | s1 | s2) % 8:
             raise ValueError(
                 "HIP attention needs 16-byte aligned Q/K/V/out with outer strides a multiple of 8"
             )
@@ -235,10 +240,10 @@ def sparse_attention(
     _check_inputs(q, k, v, kv_indices, kv_counts, global_tokens, block_size, out)
     if global_strategy not in ("flash", "triton"):
         raise ValueError("global_strategy must be flash or triton")
-    if any(
+    if any([
         isinstance(value, bool) or not isinstance(value, Integral)
         for value in (query_block_size, num_warps, num_stages)
-    ):
+    ]):
         raise TypeError("Kernel tuning arguments must be integers")
     if query_block_size not in (32, 64) or num_warps not in (4, 8) or num_stages not in (1, 2, 3, 4):
         raise ValueError("Supported tuning: query_block_size32/64, warps4/8, stages1..4")
