@@ -27,6 +27,24 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
+// A pass that reads and writes more than the 256 MB last-level cache reads its input past the caches
+// (STREAM): it cannot be there from an earlier pass, and allocating it evicts the output the next
+// kernel reads.  Measured on adaln_kernel with 3072-wide rows, three tensors in turn: 403 MB 78.0 ->
+// 68.6 us, 302 MB 59.0 -> 53.5; below the line the same loads lose whatever the caches still hold (100
+// MB 18.6 -> 21.3 us; one tensor again and again, 246 MB 39.3 -> 44.9).
+constexpr int64_t CACHE_BYTES = 256ll << 20;
+
+template <bool STREAM, typename T>
+__device__ __forceinline__ T load_once(const T* p) {
+  if constexpr (STREAM) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+template <bool STREAM, typename T>
+__device__ __forceinline__ void store_once(T* p, T v) {
+  if constexpr (STREAM) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
 // 16-bit float (bf16 or fp16) <-> fp32, round to nearest even.
 template <bool F16>
 __device__ __forceinline__ float to_f(uint16_t v) {

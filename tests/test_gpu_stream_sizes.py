@@ -1,0 +1,67 @@
+"""The HBM passes on both sides of the cache-size line, where their loads change policy: the same values.
+
+Each call past the line is compared with the same rows in calls below it: rows are independent, so
+the results are equal bit for bit."""
+
+import pytest
+import torch
+
+from tests.helpers import say
+
+pytestmark = pytest.mark.gpu
+
+CACHE = 256 << 20
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("residual", [True, False])
+def test_adaln(hip_device, dtype, residual):
+    from hilberta_amd.flux_norm import adaln_modulate
+
+    C, passes = 512, 4 if residual else 2
+    rows = CACHE // (2 * C * passes) + 37
+    gen = torch.Generator(hip_device).manual_seed(1)
+    x, y = (torch.randn(1, rows, C, device=hip_device, generator=gen).to(dtype) for _ in range(2))
+    shift, scale, gate = torch.randn(1, 3 * C, device=hip_device, generator=gen).to(dtype).chunk(3, 1)
+    say(f"case adaln past the cache size {dtype} residual={residual}")
+
+    def call(lo, hi):
+        if not residual:
+            return (adaln_modulate(x[:, lo:hi], shift, scale),)
+        r = torch.empty_like(x[:, lo:hi])
+        return r, adaln_modulate(x[:, lo:hi], shift, scale, y=y[:, lo:hi], gate=gate, x_out=r)
+
+    parts = [call(0, rows // 2), call(rows // 2, rows)]
+    for i, whole in enumerate(call(0, rows)):
+        assert torch.equal(whole, torch.cat([p[i] for p in parts], 1))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads", [5, 6, 8])
+def test_qk_prep(hip_device, dtype, heads):
+    from hilberta_amd.flux_inputs import qk_prep, qk_prep_pair
+
+    n = CACHE // (heads * 512) + 29
+    gen = torch.Generator(hip_device).manual_seed(2)
+    x = torch.randn(1, n, 2 * heads * 128, device=hip_device, generator=gen).to(dtype)
+    w = torch.rand(128, device=hip_device, generator=gen).to(dtype)
+    cos, sin = torch.rand(2, n, 128, device=hip_device, generator=gen)
+    say(f"case qk_prep past the cache size {dtype} heads={heads}")
+    whole = qk_prep_pair(None, x, heads=heads, cos=cos, sin=sin, weights=((None, w), (None, w)))
+    single = qk_prep(None, x[..., :heads * 128], heads=heads, weight_image=w, cos=cos, sin=sin)
+    assert torch.equal(single, whole[0])
+    for lo, hi in ((0, n // 3), (n // 3, 2 * n // 3), (2 * n // 3, n)):
+        part = qk_prep_pair(None, x[:, lo:hi], heads=heads, cos=cos[lo:hi], sin=sin[lo:hi],
+                            weights=((None, w), (None, w)))
+        assert torch.equal(part, whole[:, :, lo:hi])
+
+
+@pytest.mark.parametrize("row_bytes", [12, 130, 512, 6144])
+def test_gather(hip_device, row_bytes):
+    from hilberta_amd.layout import index_select_rows
+
+    rows = CACHE // (2 * row_bytes) + 53
+    x = torch.randint(-128, 128, (rows, row_bytes), dtype=torch.int8, device=hip_device)
+    index = torch.randperm(rows, device=hip_device)
+    say(f"case gather past the cache size, rows of {row_bytes} bytes")
+    assert torch.equal(index_select_rows(x, 0, index), x.index_select(0, index))
