@@ -64,3 +64,20 @@ def test_streams_keep_workspaces_apart(hip_device):
     torch.cuda.synchronize()
     _workspace.clear()
     assert set(_workspace._CACHE) == set()
+
+
+@pytest.mark.parametrize("row_bytes", [1, 3, 8, 15, 16, 17, 18, 24, 31, 33, 48, 63, 130, 4097])
+def test_row_sizes_and_alignments(hip_device, row_bytes):
+    """Rows around the 16-byte vector, at every kind of start: bytes, and bytes past the rows stay."""
+    from hilberta_amd.layout import gather_into
+
+    say(f"case gather rows of {row_bytes} bytes")
+    gen = torch.Generator().manual_seed(row_bytes)
+    for offset, gap in ((0, 0), (1, 0), (2, 5), (4, 12), (8, 8), (16, 32)):
+        flat = torch.randint(-128, 128, (offset + 300 * (row_bytes + gap),), dtype=torch.int8, generator=gen)
+        x = flat.to(hip_device)[offset:].view(300, row_bytes + gap)[:, :row_bytes]
+        index = torch.randint(0, 300, (77,), generator=gen).to(hip_device)
+        buf = torch.full((77 * row_bytes + 64 + offset,), 99, dtype=torch.int8, device=hip_device)
+        out = buf[32 + offset:32 + offset + 77 * row_bytes].view(77, row_bytes)
+        assert torch.equal(gather_into(x, 0, index, out=out), x.index_select(0, index))
+        assert (buf[:32 + offset] == 99).all() and (buf[32 + offset + 77 * row_bytes:] == 99).all()
