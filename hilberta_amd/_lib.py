@@ -66,6 +66,7 @@ SIGNATURES = {
         [_c_int, _c_int, _c_int, _c_int, _c_f32, _p, _c_i64, _c_i64, _p, _c_i64, _c_i64, _p, _c_i64,
          _p, _c_i64, _c_i64, _p, _p, _c_i64, _p, _c_i64, _c_i64, _p],
     ),
+    "hb_adaln_modulate_pair": (_c_int, [_c_int, _p, _c_int, _c_int, _c_f32, _p, _p, _p]),
     "hb_hilbert_order": (_c_int, [_c_int, _p, _p]),
     "hb_plan_layout": (_c_int, [_c_int, _c_int, _c_int, _c_int, _p, _p, _p, _p, _p, _p, _p, _p]),
     "hb_plan_scratch_bytes": (_c_i64, [_c_int, _c_int]),

@@ -34,8 +34,16 @@ struct AdaArgs {
   int64_t mod_b;
   uint16_t* out;
   int64_t out_b, out_n;
-  uint32_t rows_total, rows;
+  uint32_t rows;
   float inv_hidden, eps;
+};
+
+// Two row sets of one shape (the image and text rows of a double-stream block) share a launch: 512
+// text rows alone are 6-9 us of a mostly idle chip (a two-block transformer at 1024 px 0.5-0.8 % faster).
+// The first `rows0` of `total` rows are a[0]'s.
+struct AdaPair {
+  AdaArgs a[2];
+  uint32_t rows0, total;
 };
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -44,11 +52,16 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-template <bool F16, int NV, bool STREAM>
-__global__ __launch_bounds__(256) void adaln_kernel(AdaArgs a) {
+template <bool F16, int NV, bool STREAM, bool PAIR>
+__global__ __launch_bounds__(256) void adaln_kernel(AdaPair p) {
 #pragma clang fp contract(off)
-  const uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
-  if (row >= a.rows_total) return;  // the whole wave leaves together
+  uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
+  if (row >= p.total) return;  // the whole wave leaves together
+  // (a wave lives for one row, so a single set's operands are not made to wait for the choice: 2 % of
+  // a 403 MB call)
+  const bool second = PAIR && (uint32_t)uniform(row) >= p.rows0;
+  const AdaArgs& a = p.a[second];
+  if (second) row -= p.rows0;
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t b = row / a.rows;
   const uint32_t i = row - b * a.rows;
@@ -116,26 +129,98 @@ __global__ __launch_bounds__(256) void adaln_kernel(AdaArgs a) {
   }
 }
 
-template <bool F16, bool STREAM>
-int launch(const AdaArgs& a, int nv, hipStream_t st) {
-  const dim3 grid((a.rows_total + 3) / 4), block(256);
+template <bool F16, bool STREAM, bool PAIR>
+int launch(const AdaPair& a, int nv, hipStream_t st) {
+  const dim3 grid((a.total + 3) / 4), block(256);
   switch (nv) {
-    case 1: hipLaunchKernelGGL((adaln_kernel<F16, 1, STREAM>), grid, block, 0, st, a); break;
-    case 2: hipLaunchKernelGGL((adaln_kernel<F16, 2, STREAM>), grid, block, 0, st, a); break;
-    case 3: hipLaunchKernelGGL((adaln_kernel<F16, 3, STREAM>), grid, block, 0, st, a); break;
-    case 4: hipLaunchKernelGGL((adaln_kernel<F16, 4, STREAM>), grid, block, 0, st, a); break;
-    case 6: hipLaunchKernelGGL((adaln_kernel<F16, 6, STREAM>), grid, block, 0, st, a); break;
-    case 8: hipLaunchKernelGGL((adaln_kernel<F16, 8, STREAM>), grid, block, 0, st, a); break;
+    case 1: hipLaunchKernelGGL((adaln_kernel<F16, 1, STREAM, PAIR>), grid, block, 0, st, a); break;
+    case 2: hipLaunchKernelGGL((adaln_kernel<F16, 2, STREAM, PAIR>), grid, block, 0, st, a); break;
+    case 3: hipLaunchKernelGGL((adaln_kernel<F16, 3, STREAM, PAIR>), grid, block, 0, st, a); break;
+    case 4: hipLaunchKernelGGL((adaln_kernel<F16, 4, STREAM, PAIR>), grid, block, 0, st, a); break;
+    case 6: hipLaunchKernelGGL((adaln_kernel<F16, 6, STREAM, PAIR>), grid, block, 0, st, a); break;
+    case 8: hipLaunchKernelGGL((adaln_kernel<F16, 8, STREAM, PAIR>), grid, block, 0, st, a); break;
     default: set_error("hidden must be 512, 1024, 1536, 2048, 3072 or 4096"); return HB_EINVAL;
   }
   HB_HIP(hipGetLastError());
   return HB_OK;
 }
 
+template <bool F16, bool STREAM>
+int launch_sets(const AdaPair& p, int nv, int count, hipStream_t st) {
+  return count == 2 ? launch<F16, STREAM, true>(p, nv, st) : launch<F16, STREAM, false>(p, nv, st);
+}
+
 }  // namespace
 }  // namespace hb
 
 using namespace hb;
+
+namespace {
+
+// Operands of one row set, as the entry points take them.
+struct Operands {
+  const void *x, *y, *gate;
+  void* x_out;
+  const void *shift, *scale;
+  void* out;
+  int64_t x_b, x_n, y_b, y_n, gate_b, xo_b, xo_n, mod_b, out_b, out_n;
+};
+
+int modulate(int count, int32_t batch, const int32_t* rows, int32_t hidden, int32_t dtype, float eps,
+             const Operands* sets, hipStream_t stream) {
+  AdaPair p = {};
+  int64_t total = 0, bytes = 0;
+  for (int i = 0; i < count; ++i) {
+    const Operands& o = sets[i];
+    HB_REQUIRE(batch > 0 && rows[i] > 0, "batch and rows must be positive");
+    total += (int64_t)batch * rows[i];
+    HB_REQUIRE(total < (1ll << 31), "too many rows for one launch");
+    HB_REQUIRE(hidden > 0 && hidden % 512 == 0, "hidden must be a multiple of 512 (got %d)", hidden);
+    HB_REQUIRE(dtype == HB_DTYPE_BF16 || dtype == HB_DTYPE_F16, "dtype must be bf16 or fp16");
+    HB_REQUIRE(eps > 0.f, "eps must be positive");
+    HB_REQUIRE(o.x && o.shift && o.scale && o.out, "null pointer argument");
+    HB_REQUIRE(!o.y || o.gate, "a residual update needs its gate");
+    HB_REQUIRE(!o.x_out || o.y, "x_out is written only with a residual update");
+    const void* ptrs[7] = {o.x, o.y, o.gate, o.x_out, o.shift, o.scale, o.out};
+    for (int k = 0; k < 7; ++k)
+      HB_REQUIRE(((uintptr_t)ptrs[k] & 15) == 0, "every pointer must be 16-byte aligned");
+    const int64_t strides[10] = {o.x_b, o.x_n, o.y_b, o.y_n, o.gate_b, o.xo_b, o.xo_n, o.mod_b, o.out_b, o.out_n};
+    for (int k = 0; k < 10; ++k)
+      HB_REQUIRE(strides[k] >= 0 && strides[k] % 8 == 0, "strides must be non-negative multiples of 8");
+    // x (and y) in, the residual (when stored) and the rows out
+    bytes += (int64_t)batch * rows[i] * hidden * 2 * (2 + (o.y != nullptr) + (o.x_out != nullptr));
+    AdaArgs& a = p.a[i];
+    a.x = (const uint16_t*)o.x;
+    a.x_b = o.x_b;
+    a.x_n = o.x_n;
+    a.y = (const uint16_t*)o.y;
+    a.y_b = o.y_b;
+    a.y_n = o.y_n;
+    a.gate = (const uint16_t*)o.gate;
+    a.gate_b = o.gate_b;
+    a.x_out = (uint16_t*)o.x_out;
+    a.xo_b = o.xo_b;
+    a.xo_n = o.xo_n;
+    a.shift = (const uint16_t*)o.shift;
+    a.scale = (const uint16_t*)o.scale;
+    a.mod_b = o.mod_b;
+    a.out = (uint16_t*)o.out;
+    a.out_b = o.out_b;
+    a.out_n = o.out_n;
+    a.rows = (uint32_t)rows[i];
+    a.inv_hidden = 1.f / (float)hidden;
+    a.eps = eps;
+    if (i == 0) p.rows0 = (uint32_t)total;
+  }
+  p.total = (uint32_t)total;
+  const int nv = hidden / 512;
+  const bool stream_in = bytes > CACHE_BYTES;
+  if (dtype == HB_DTYPE_F16)
+    return stream_in ? launch_sets<true, true>(p, nv, count, stream) : launch_sets<true, false>(p, nv, count, stream);
+  return stream_in ? launch_sets<false, true>(p, nv, count, stream) : launch_sets<false, false>(p, nv, count, stream);
+}
+
+}  // namespace
 
 extern "C" int hb_adaln_modulate(int32_t batch, int32_t rows, int32_t hidden, int32_t dtype,
                                  float eps, const void* x, int64_t x_batch_stride,
@@ -146,49 +231,21 @@ extern "C" int hb_adaln_modulate(int32_t batch, int32_t rows, int32_t hidden, in
                                  const void* shift, const void* scale, int64_t mod_batch_stride,
                                  void* out, int64_t out_batch_stride, int64_t out_row_stride,
                                  hb_stream_t stream) {
-  HB_REQUIRE(batch > 0 && rows > 0, "batch and rows must be positive");
-  HB_REQUIRE((int64_t)batch * rows < (1ll << 31), "too many rows for one launch");
-  HB_REQUIRE(hidden > 0 && hidden % 512 == 0, "hidden must be a multiple of 512 (got %d)", hidden);
-  HB_REQUIRE(dtype == HB_DTYPE_BF16 || dtype == HB_DTYPE_F16, "dtype must be bf16 or fp16");
-  HB_REQUIRE(eps > 0.f, "eps must be positive");
-  HB_REQUIRE(x && shift && scale && out, "null pointer argument");
-  HB_REQUIRE(!y || gate, "a residual update needs its gate");
-  HB_REQUIRE(!x_out || y, "x_out is written only with a residual update");
-  const void* ptrs[7] = {x, y, gate, x_out, shift, scale, out};
-  for (int k = 0; k < 7; ++k)
-    HB_REQUIRE(((uintptr_t)ptrs[k] & 15) == 0, "every pointer must be 16-byte aligned");
-  const int64_t strides[10] = {x_batch_stride, x_row_stride, y_batch_stride, y_row_stride,
-                               gate_batch_stride, x_out_batch_stride, x_out_row_stride,
-                               mod_batch_stride, out_batch_stride, out_row_stride};
-  for (int k = 0; k < 10; ++k)
-    HB_REQUIRE(strides[k] >= 0 && strides[k] % 8 == 0, "strides must be non-negative multiples of 8");
-  AdaArgs a;
-  a.x = (const uint16_t*)x;
-  a.x_b = x_batch_stride;
-  a.x_n = x_row_stride;
-  a.y = (const uint16_t*)y;
-  a.y_b = y_batch_stride;
-  a.y_n = y_row_stride;
-  a.gate = (const uint16_t*)gate;
-  a.gate_b = gate_batch_stride;
-  a.x_out = (uint16_t*)x_out;
-  a.xo_b = x_out_batch_stride;
-  a.xo_n = x_out_row_stride;
-  a.shift = (const uint16_t*)shift;
-  a.scale = (const uint16_t*)scale;
-  a.mod_b = mod_batch_stride;
-  a.out = (uint16_t*)out;
-  a.out_b = out_batch_stride;
-  a.out_n = out_row_stride;
-  a.rows_total = (uint32_t)(batch * rows);
-  a.rows = (uint32_t)rows;
-  a.inv_hidden = 1.f / (float)hidden;
-  a.eps = eps;
-  const int nv = hidden / 512;
-  // x (and y) in, the residual (when stored) and the rows out
-  const bool stream_in = (int64_t)batch * rows * hidden * 2 * (2 + (y != nullptr) + (x_out != nullptr)) > CACHE_BYTES;
-  const hipStream_t st = (hipStream_t)stream;
-  if (dtype == HB_DTYPE_F16)
-    return stream_in ? launch<true, true>(a, nv, st) : launch<true, false>(a, nv, st);
-  return stream_in ? launch<false, true>(a, nv, st) : launch<false, false>(a, nv, st);
+  const Operands o = {x, y, gate, x_out, shift, scale, out, x_batch_stride, x_row_stride,
+                      y_batch_stride, y_row_stride, gate_batch_stride, x_out_batch_stride,
+                      x_out_row_stride, mod_batch_stride, out_batch_stride, out_row_stride};
+  return modulate(1, batch, &rows, hidden, dtype, eps, &o, stream);
+}
+
+extern "C" int hb_adaln_modulate_pair(int32_t batch, const int32_t* rows, int32_t hidden,
+                                      int32_t dtype, float eps, void* const* pointers,
+                                      const int64_t* strides, hb_stream_t stream) {
+  HB_REQUIRE(rows && pointers && strides, "null pointer argument");
+  Operands o[2];
+  for (int i = 0; i < 2; ++i) {
+    void* const* q = pointers + 7 * i;
+    const int64_t* s = strides + 10 * i;
+    o[i] = {q[0], q[1], q[2], q[3], q[4], q[5], q[6], s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], s[8], s[9]};
+  }
+  return modulate(2, batch, rows, hidden, dtype, eps, o, stream);
 }

@@ -43,7 +43,7 @@ import torch.nn.functional as F
 
 from .flux_cond import embed, linear_layers, timestep_projection  # noqa: F401
 from .flux_inputs import qk_prep_pair, rotary_tables
-from .flux_norm import adaln_modulate
+from .flux_norm import adaln_modulate, adaln_modulate_pair
 from .layout import index_select_rows
 
 
@@ -345,8 +345,8 @@ class FluxTransformer:
         ax = F.linear(o[:, T:], *w["out_x"])
         ac = F.linear(o[:, :T], *w["out_c"])
         del o
-        xn = adaln_modulate(x, sx2, scx2, y=ax, gate=gx, x_out=x, eps=s.eps)
-        cn = adaln_modulate(c, sc2, scc2, y=ac, gate=gc, x_out=c, eps=s.eps)
+        xn, cn = adaln_modulate_pair(dict(x=x, shift=sx2, scale=scx2, y=ax, gate=gx, x_out=x),
+                                     dict(x=c, shift=sc2, scale=scc2, y=ac, gate=gc, x_out=c), eps=s.eps)
         del ax, ac
         (w1, b1), (w2, b2) = w["ff_x"]
         fx = F.linear(_gelu_linear(xn, w1, b1), w2, b2)
@@ -354,13 +354,14 @@ class FluxTransformer:
         fc = F.linear(_gelu_linear(cn, w1, b1), w2, b2)
         if joint_out is None:
             (nsx, nscx), (nsc, nscc) = next_mods
-            xn = adaln_modulate(x, nsx, nscx, y=fx, gate=gx2, x_out=x, eps=s.eps)
-            cn = adaln_modulate(c, nsc, nscc, y=fc, gate=gc2, x_out=c, eps=s.eps)
+            xn, cn = adaln_modulate_pair(dict(x=x, shift=nsx, scale=nscx, y=fx, gate=gx2, x_out=x),
+                                         dict(x=c, shift=nsc, scale=nscc, y=fc, gate=gc2, x_out=c), eps=s.eps)
             return x, xn, c, cn
         h, hn = joint_out
         nshift, nscale = next_mods
-        adaln_modulate(x, nshift, nscale, y=fx, gate=gx2, x_out=h[:, T:], out=hn[:, T:], eps=s.eps)
-        adaln_modulate(c, nshift, nscale, y=fc, gate=gc2, x_out=h[:, :T], out=hn[:, :T], eps=s.eps)
+        mod = dict(shift=nshift, scale=nscale)
+        adaln_modulate_pair(dict(mod, x=x, y=fx, gate=gx2, x_out=h[:, T:], out=hn[:, T:]),
+                            dict(mod, x=c, y=fc, gate=gc2, x_out=h[:, :T], out=hn[:, :T]), eps=s.eps)
         return None
 
     def _single_block(self, w, mods, h, hn, T, cos, sin, attention, layer, next_mods):
@@ -434,8 +435,7 @@ class FluxTransformer:
         x = F.linear(hidden_states.to(self.dtype), *self.x_embedder)
         c = F.linear(encoder_hidden_states.to(self.dtype), *self.context_embedder)
         (sx, scx, *_), (sc, scc, *_) = double_mods[0]
-        xn = adaln_modulate(x, sx, scx, eps=s.eps)
-        cn = adaln_modulate(c, sc, scc, eps=s.eps)
+        xn, cn = adaln_modulate_pair(dict(x=x, shift=sx, scale=scx), dict(x=c, shift=sc, scale=scc), eps=s.eps)
         h = torch.empty(B, N, s.hidden, device=x.device, dtype=x.dtype)
         hn = torch.empty_like(h)
         for i, w in enumerate(self.double):

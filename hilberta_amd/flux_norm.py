@@ -11,6 +11,8 @@ AdaLayerNormZero / AdaLayerNormZeroSingle / AdaLayerNormContinuous) run as separ
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -24,9 +26,8 @@ def _rows(t, name, B, R, C):
     return t.stride(0), t.stride(1)
 
 
-def adaln_modulate(x, shift, scale, *, y=None, gate=None, x_out=None, out=None, eps=1e-6):
-    """x [B, rows, hidden]; shift / scale / gate [B, hidden] (views with a contiguous last dim,
-    e.g. chunks of one modulation projection); y like x.  Returns out [B, rows, hidden]."""
+def _operands(x, shift, scale, y, gate, x_out, out):
+    """Checked (pointers, strides, out) of one row set, in the order of hb_adaln_modulate_pair."""
     _lib.require_gpu(x)
     if x.dtype not in _DTYPES:
         raise ValueError("adaln_modulate takes bf16 or fp16 rows")
@@ -57,11 +58,37 @@ def adaln_modulate(x, shift, scale, *, y=None, gate=None, x_out=None, out=None, 
     tensors.append(out)
     if any(t.device != x.device or t.dtype != x.dtype for t in tensors):
         raise ValueError("all tensors must share x's device and dtype")
-    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    pointers = [None if t is None else t.data_ptr() for t in (x, y, gate, x_out, shift, scale, out)]
+    gate_b = gate.stride(0) if gate is not None else 0
+    return pointers, [xb, xn, yb, yn, gate_b, ob, on, mod_b, pb, pn], out
+
+
+def adaln_modulate(x, shift, scale, *, y=None, gate=None, x_out=None, out=None, eps=1e-6):
+    """x [B, rows, hidden]; shift / scale / gate [B, hidden] (views with a contiguous last dim,
+    e.g. chunks of one modulation projection); y like x.  Returns out [B, rows, hidden]."""
+    (px, py, pg, po, psh, psc, pout), (xb, xn, yb, yn, gb, ob, on, mb, pb, pn), out = _operands(
+        x, shift, scale, y, gate, x_out, out)
+    B, R, C = x.shape
     rc = _lib.load().hb_adaln_modulate(
-        B, R, C, _DTYPES[x.dtype], float(eps), x.data_ptr(), xb, xn, ptr(y), yb, yn, ptr(gate),
-        gate.stride(0) if gate is not None else 0, ptr(x_out), ob, on, shift.data_ptr(), scale.data_ptr(), mod_b, out.data_ptr(), pb, pn,
-        _lib.stream_ptr(x.device),
+        B, R, C, _DTYPES[x.dtype], float(eps), px, xb, xn, py, yb, yn, pg, gb, po, ob, on, psh, psc,
+        mb, pout, pb, pn, _lib.stream_ptr(x.device),
     )
     _lib.check(rc, "hb_adaln_modulate")
     return out
+
+
+def adaln_modulate_pair(first, second, *, eps=1e-6):
+    """adaln_modulate of two row sets in one launch (the image and text streams of a double block):
+    ``first`` and ``second`` are its arguments as dicts, of one batch, hidden size, dtype and device.
+    Returns both outputs."""
+    sets = [_operands(s["x"], s["shift"], s["scale"], s.get("y"), s.get("gate"), s.get("x_out"),
+                      s.get("out")) for s in (first, second)]
+    a, b = first["x"], second["x"]
+    if a.shape[0] != b.shape[0] or a.shape[2] != b.shape[2] or a.dtype != b.dtype or a.device != b.device:
+        raise ValueError("both row sets must share batch, hidden size, dtype and device")
+    rc = _lib.load().hb_adaln_modulate_pair(
+        a.shape[0], (ctypes.c_int32 * 2)(a.shape[1], b.shape[1]), a.shape[2], _DTYPES[a.dtype], float(eps),
+        (ctypes.c_void_p * 14)(*sets[0][0], *sets[1][0]), (ctypes.c_int64 * 20)(*sets[0][1], *sets[1][1]),
+        _lib.stream_ptr(a.device))
+    _lib.check(rc, "hb_adaln_modulate_pair")
+    return sets[0][2], sets[1][2]

@@ -206,6 +206,14 @@ int hb_adaln_modulate(int32_t batch, int32_t rows, int32_t hidden, int32_t dtype
                       const void* scale, int64_t mod_batch_stride, void* out,
                       int64_t out_batch_stride, int64_t out_row_stride, hb_stream_t stream);
 
+/* hb_adaln_modulate of two row sets of one batch, hidden size and type in one launch (the image and text
+ * streams of a double block).  Host arrays, set 0 then set 1: rows [2]; pointers [2 x 7] {x, y, gate,
+ * x_out, shift, scale, out} (y, gate and x_out may be NULL, as above); strides [2 x 10] {x batch, x row, y
+ * batch, y row, gate batch, x_out batch, x_out row, mod batch, out batch, out row}. */
+int hb_adaln_modulate_pair(int32_t batch, const int32_t* rows, int32_t hidden, int32_t dtype,
+                           float eps, void* const* pointers, const int64_t* strides,
+                           hb_stream_t stream);
+
 /* ---------------------------------------------------------------- (b) block tables
  * Hilbert order of a grid_size x grid_size raster (reference hilberta/geometry.py:6-25). */
 int hb_hilbert_order(int32_t grid_size, int64_t* out, hb_stream_t stream);

@@ -96,3 +96,29 @@ def test_argument_errors(hip_device):
         adaln_modulate(x, m, m, x_out=x)
     with pytest.raises(ValueError):
         adaln_modulate(x[..., :1000], m[:, :1000], m[:, :1000])
+
+
+@pytest.mark.parametrize("rows", [(1, 1), (3, 2), (4, 5), (129, 7), (5, 1030)])
+@pytest.mark.parametrize("batch", [1, 3])
+def test_pair_equals_two_calls(hip_device, rows, batch):
+    """Two row sets in one launch: bitwise the two calls, at every split of a workgroup's four rows."""
+    from hilberta_amd.flux_norm import adaln_modulate, adaln_modulate_pair
+
+    gen = torch.Generator("cpu").manual_seed(sum(rows))
+    new = lambda *s: torch.randn(*s, generator=gen).to(torch.bfloat16).to(hip_device)  # noqa: E731
+    say(f"case adaln pair rows={rows} batch={batch}")
+    for residual in ((True, True), (True, False), (False, False)):
+        sets, apart = [], []
+        for r, res in zip(rows, residual):
+            shift, scale, gate = new(batch, 3 * 512).chunk(3, 1)
+            x = new(batch, r + 2, 512)[:, 1:-1]
+            y = new(batch, r, 512) if res else None
+            kw = dict(y=y, gate=gate, x_out=torch.empty(batch, r, 512, dtype=x.dtype, device=x.device)) if res else {}
+            sets.append(dict(x=x, shift=shift, scale=scale, **kw))
+            ref = dict(kw, x_out=torch.empty_like(kw["x_out"])) if res else {}
+            apart.append((adaln_modulate(x, shift, scale, **ref), ref.get("x_out")))
+        for got, s, (ref, ref_x) in zip(adaln_modulate_pair(*sets), sets, apart):
+            assert torch.equal(got, ref) and (ref_x is None or torch.equal(s["x_out"], ref_x))
+    bad = dict(x=new(batch + 1, 2, 512), shift=new(batch + 1, 512), scale=new(batch + 1, 512))
+    with pytest.raises(ValueError):
+        adaln_modulate_pair(sets[0], bad)
