@@ -20,59 +20,66 @@ from . import _lib
 _DTYPES = {torch.bfloat16: 0, torch.float16: 1}
 
 
-def _rows(t, name, B, R, C):
-    if t.ndim != 3 or t.shape != (B, R, C) or t.stride(-1) != 1:
+def _strides(t, name, shape, dtype, device):
+    """(batch, row) strides of one [B, rows, hidden] operand, and whether it is of x's kind."""
+    st = t.stride()
+    if t.shape != shape or st[2] != 1:
         raise ValueError(f"{name} must be [B, rows, hidden] with a contiguous last dimension")
-    return t.stride(0), t.stride(1)
+    return st[0], st[1], t.dtype == dtype and t.device == device
 
 
 def _operands(x, shift, scale, y, gate, x_out, out):
-    """Checked (pointers, strides, out) of one row set, in the order of hb_adaln_modulate_pair."""
-    _lib.require_gpu(x)
-    if x.dtype not in _DTYPES:
+    """Checked operands of one row set: seven pointers and ten strides in the order of
+    hb_adaln_modulate_pair, the sizes, and the output.  (A short call is as long as these checks, so
+    each tensor attribute is read once.)"""
+    if not (isinstance(x, torch.Tensor) and x.is_cuda):
+        _lib.require_gpu(x)
+    dtype, device, shape = x.dtype, x.device, x.shape
+    if dtype not in _DTYPES:
         raise ValueError("adaln_modulate takes bf16 or fp16 rows")
-    B, R, C = x.shape if x.ndim == 3 else (0, 0, 0)
-    xb, xn = _rows(x, "x", B, R, C)
-    yb = yn = ob = on = 0
+    if len(shape) != 3:
+        raise ValueError("x must be [B, rows, hidden] with a contiguous last dimension")
+    xb, xn, same = _strides(x, "x", shape, dtype, device)
+    yb = yn = gate_b = ob = on = 0
+    py = pg = po = None
     if (y is None) != (gate is None):
         raise ValueError("y and gate are given together")
     if x_out is not None and y is None:
         raise ValueError("x_out is written only with a residual update")
-    mods = [shift, scale] + ([gate] if gate is not None else [])
-    for m in mods:
-        if m.ndim != 2 or m.shape != (B, C) or m.stride(-1) != 1 or m.dtype != x.dtype:
+    row = (shape[0], shape[2])
+    for m in (shift, scale) if gate is None else (shift, scale, gate):
+        if m.shape != row or m.stride(1) != 1 or m.dtype != dtype:
             raise ValueError("shift/scale/gate must be [B, hidden] views with a contiguous last dim")
+        same = same and m.device == device
     mod_b = shift.stride(0)
     if scale.stride(0) != mod_b:
         raise ValueError("shift and scale must share one batch stride")
-    tensors = [x] + mods
     if y is not None:
-        yb, yn = _rows(y, "y", B, R, C)
-        tensors.append(y)
+        yb, yn, ok = _strides(y, "y", shape, dtype, device)
+        same, py, pg, gate_b = same and ok, y.data_ptr(), gate.data_ptr(), gate.stride(0)
     if x_out is not None:
-        ob, on = _rows(x_out, "x_out", B, R, C)
-        tensors.append(x_out)
+        ob, on, ok = _strides(x_out, "x_out", shape, dtype, device)
+        same, po = same and ok, x_out.data_ptr()
     if out is None:
-        out = torch.empty(B, R, C, dtype=x.dtype, device=x.device)
-    pb, pn = _rows(out, "out", B, R, C)
-    tensors.append(out)
-    if any(t.device != x.device or t.dtype != x.dtype for t in tensors):
+        out = torch.empty(shape, dtype=dtype, device=device)
+        pb, pn = shape[1] * shape[2], shape[2]
+    else:
+        pb, pn, ok = _strides(out, "out", shape, dtype, device)
+        same = same and ok
+    if not same:
         raise ValueError("all tensors must share x's device and dtype")
-    pointers = [None if t is None else t.data_ptr() for t in (x, y, gate, x_out, shift, scale, out)]
-    gate_b = gate.stride(0) if gate is not None else 0
-    return pointers, [xb, xn, yb, yn, gate_b, ob, on, mod_b, pb, pn], out
+    return ((x.data_ptr(), py, pg, po, shift.data_ptr(), scale.data_ptr(), out.data_ptr()),
+            (xb, xn, yb, yn, gate_b, ob, on, mod_b, pb, pn), (*shape, _DTYPES[dtype], device), out)
 
 
 def adaln_modulate(x, shift, scale, *, y=None, gate=None, x_out=None, out=None, eps=1e-6):
     """x [B, rows, hidden]; shift / scale / gate [B, hidden] (views with a contiguous last dim,
     e.g. chunks of one modulation projection); y like x.  Returns out [B, rows, hidden]."""
-    (px, py, pg, po, psh, psc, pout), (xb, xn, yb, yn, gb, ob, on, mb, pb, pn), out = _operands(
-        x, shift, scale, y, gate, x_out, out)
-    B, R, C = x.shape
+    (px, py, pg, po, psh, psc, pout), (xb, xn, yb, yn, gb, ob, on, mb, pb, pn), (B, R, C, code, device), out = \
+        _operands(x, shift, scale, y, gate, x_out, out)
     rc = _lib.load().hb_adaln_modulate(
-        B, R, C, _DTYPES[x.dtype], float(eps), px, xb, xn, py, yb, yn, pg, gb, po, ob, on, psh, psc,
-        mb, pout, pb, pn, _lib.stream_ptr(x.device),
-    )
+        B, R, C, code, float(eps), px, xb, xn, py, yb, yn, pg, gb, po, ob, on, psh, psc, mb, pout, pb, pn,
+        _lib.stream_ptr(device))
     _lib.check(rc, "hb_adaln_modulate")
     return out
 
@@ -83,12 +90,11 @@ def adaln_modulate_pair(first, second, *, eps=1e-6):
     Returns both outputs."""
     sets = [_operands(s["x"], s["shift"], s["scale"], s.get("y"), s.get("gate"), s.get("x_out"),
                       s.get("out")) for s in (first, second)]
-    a, b = first["x"], second["x"]
-    if a.shape[0] != b.shape[0] or a.shape[2] != b.shape[2] or a.dtype != b.dtype or a.device != b.device:
+    (pa, sa, (B, ra, C, code, device), out_a), (pb, sb, (Bb, rb, Cb, codeb, deviceb), out_b) = sets
+    if (B, C, code, device) != (Bb, Cb, codeb, deviceb):
         raise ValueError("both row sets must share batch, hidden size, dtype and device")
     rc = _lib.load().hb_adaln_modulate_pair(
-        a.shape[0], (ctypes.c_int32 * 2)(a.shape[1], b.shape[1]), a.shape[2], _DTYPES[a.dtype], float(eps),
-        (ctypes.c_void_p * 14)(*sets[0][0], *sets[1][0]), (ctypes.c_int64 * 20)(*sets[0][1], *sets[1][1]),
-        _lib.stream_ptr(a.device))
+        B, (ctypes.c_int32 * 2)(ra, rb), C, code, float(eps), (ctypes.c_void_p * 14)(*pa, *pb),
+        (ctypes.c_int64 * 20)(*sa, *sb), _lib.stream_ptr(device))
     _lib.check(rc, "hb_adaln_modulate_pair")
-    return sets[0][2], sets[1][2]
+    return out_a, out_b
