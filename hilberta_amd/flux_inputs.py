@@ -30,11 +30,13 @@ _ID_DTYPES = (torch.float32, torch.bfloat16, torch.float16, torch.float64, torch
 
 
 def rotary_tables(ids, theta=THETA, axes_dim=AXES_DIM):
-    """(cos, sin) float32 [N, 128] for position ids [N, 3] (diffusers 0.36.0 FluxPosEmbed: float64
-    angles pos * theta^(-2j/d) per axis, each value repeated for the pair, axes concatenated)."""
+    """(cos, sin) float32 [N, 128] for position ids [N, axes], three in FLUX (diffusers 0.36.0
+    FluxPosEmbed: float64 angles pos * theta^(-2j/d) per axis, each value repeated for the pair, axes
+    concatenated)."""
     if ids.ndim != 2 or ids.shape[1] != len(axes_dim) or sum(axes_dim) != HEAD_DIM:
         raise ValueError("ids must be [N, 3] and the axes must add up to 128")
-    if (_lib.is_plain(ids) and ids.dtype in _ID_DTYPES and type(theta) in (int, float)
+    # (the kernel walks rows of three ids; one, two or four and more axes are composed)
+    if (len(axes_dim) == 3 and _lib.is_plain(ids) and ids.dtype in _ID_DTYPES and type(theta) in (int, float)
             and 0 < theta < math.inf and all(type(d) is int and d >= 0 and d % 2 == 0 for d in axes_dim)):
         return _rotary_tables_hip(ids, float(theta), axes_dim)
     pos = ids.to(torch.float32).to(torch.float64)

@@ -40,3 +40,13 @@ def test_other_forms(hip_device):
     assert [t.shape for t in rotary_tables(torch.zeros(0, 3, device=hip_device))] == [(0, 128)] * 2
     x = ids[:, :3].float().to(hip_device).requires_grad_()
     assert rotary_tables(x)[0].requires_grad   # the composed path serves differentiation
+
+
+@pytest.mark.parametrize("axes", [(128,), (64, 64), (32, 32, 32, 32)])
+def test_other_axis_counts(hip_device, axes):
+    """Composed: the kernel reads rows of three ids."""
+    gen = torch.Generator().manual_seed(len(axes))
+    ids = torch.randint(0, 257, (77, len(axes)), generator=gen).float()
+    say(f"case rotary axes={axes}")
+    for g, r in zip(rotary_tables(ids.to(hip_device), axes_dim=axes), F.rotary_tables(ids, axes_dim=axes)):
+        assert g.shape == (77, 128) and (g.cpu() - r).abs().max() <= 2 ** -24
