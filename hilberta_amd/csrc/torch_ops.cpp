@@ -8,8 +8,10 @@
 // implementations and the CPU kernel of pair_rows, which is plan setup, are in hilberta_amd/ops.py.
 #include <ATen/ATen.h>
 #include <ATen/DeviceGuard.h>
+#include <ATen/core/LegacyTypeDispatch.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
+#include <torch/csrc/autograd/variable.h>
 #include <torch/library.h>
 
 #include <limits>
@@ -267,6 +269,46 @@ Tensor gather_rows(const Tensor& input, int64_t dim, const Tensor& index) {
   return out;
 }
 
+// The attention operators return nothing and write `out` and `lse`, which torch's own boxed fallbacks
+// overlook: they look after returned tensors only.
+
+// No derivative is recorded (the entry points refuse inputs that need one); a transform that takes one
+// is refused, as torch refuses an autograd.Function in one, for it would get zeros.
+void attention_autograd(const c10::OperatorHandle& op, c10::DispatchKeySet keys, torch::jit::Stack* stack) {
+  const size_t count = op.schema().arguments().size();
+  // (included for as long as any torch.func transform is active)
+  const bool transformed = at::GradMode::is_enabled() &&
+                           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerBackMode);
+  for (const c10::IValue& value : torch::jit::last(stack, count)) {
+    if (!value.isTensor() || !value.toTensor().defined()) continue;
+    const Tensor& t = value.toTensor();
+    TORCH_CHECK_NOT_IMPLEMENTED(!t._fw_grad(/*level=*/0).defined(), "Trying to use forward AD with ",
+                                op.schema().name(), " that does not support it.");
+    TORCH_CHECK(!(transformed && t.requires_grad()), op.schema().name(), " has no derivative for torch.func transforms");
+  }
+  const at::AutoDispatchBelowAutograd below;
+  op.redispatchBoxed(keys & c10::after_autograd_keyset, stack);
+}
+
+// A tensor saved for a backward and then overwritten here has to fail that backward: every written
+// argument's version counts up.
+void attention_writes(const c10::OperatorHandle& op, c10::DispatchKeySet keys, torch::jit::Stack* stack) {
+  const auto& arguments = op.schema().arguments();
+  const auto values = torch::jit::last(stack, arguments.size());
+  c10::SmallVector<Tensor, 2> written;
+  for (size_t i = 0; i < arguments.size(); ++i) {
+    const c10::AliasInfo* alias = arguments[i].alias_info();
+    if (alias && alias->isWrite() && values[i].isTensor() && values[i].toTensor().defined())
+      written.push_back(values[i].toTensor());
+  }
+  {
+    const at::AutoDispatchBelowADInplaceOrView below;
+    op.redispatchBoxed(keys & c10::after_ADInplaceOrView_keyset, stack);
+  }
+  for (const Tensor& t : written)
+    if (!t.is_inference()) torch::autograd::impl::bump_version(t);
+}
+
 }  // namespace
 
 TORCH_LIBRARY(hilberta_hip, m) {
@@ -298,13 +340,15 @@ TORCH_LIBRARY_IMPL(hilberta_hip, CompositeExplicitAutograd, m) {
   m.impl("_clear_workspaces", clear_workspaces);
 }
 
-// Inference operators: a differentiated call fails in its backward, in-place writes count.
+// gather_rows and pair_rows: a differentiated call fails in its backward.
 TORCH_LIBRARY_IMPL(hilberta_hip, Autograd, m) {
-  for (const char* name : {"paired_fwd", "sparse_fwd", "pair_rows", "gather_rows"})
+  for (const char* name : {"pair_rows", "gather_rows"})
     m.impl(name, torch::autograd::autogradNotImplementedFallback());
+  for (const char* name : {"paired_fwd", "sparse_fwd"})
+    m.impl(name, torch::CppFunction::makeFromBoxedFunction<&attention_autograd>());
 }
 
 TORCH_LIBRARY_IMPL(hilberta_hip, ADInplaceOrView, m) {
   for (const char* name : {"paired_fwd", "sparse_fwd"})
-    m.impl(name, torch::autograd::autogradNotImplementedInplaceOrViewFallback());
+    m.impl(name, torch::CppFunction::makeFromBoxedFunction<&attention_writes>());
 }

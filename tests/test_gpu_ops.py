@@ -93,3 +93,21 @@ def test_op_call_equals_direct_c_abi_launch(case):
     x = torch.randn(1, 4096, 3072, device=q.device).to(torch.bfloat16)
     order = torch.from_numpy(np.random.default_rng(1).permutation(4096)).to(q.device)
     assert torch.equal(OPS.gather_rows(x, 1, order), x.index_select(1, order))
+
+
+def test_entry_points_count_their_writes(case):
+    """paired_attention and sparse_attention mark ``out`` and ``lse`` as written."""
+    from hilberta_amd.paired_kernel import paired_attention
+    from hilberta_amd.sparse_kernel import sparse_attention
+
+    plan, q, k, v, meta, ids, counts = case
+    say("case version counters of out and lse")
+    out, lse = torch.empty_like(q), torch.empty(q.shape[:3], dtype=torch.float32, device=q.device)
+    saved = torch.ones(q.shape[:3], device=q.device, requires_grad=True)
+    y = (lse.zero_() * saved).sum()
+    before = out._version, lse._version
+    paired_attention(q, k, v, meta, out=out, lse=lse)
+    sparse_attention(q, k, v, ids, counts, global_tokens=plan["global_tokens"], out=out, lse=lse)
+    assert (out._version, lse._version) == (before[0] + 2, before[1] + 2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward()
