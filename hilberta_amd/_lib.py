@@ -163,10 +163,12 @@ def is_plain(*tensors) -> bool:
     """True for ordinary device tensors outside any transform: no subclass (fake tensors), no
     dispatch or function mode, tracing or torch.func level, no forward- or reverse-mode gradient.
     Calls that composed torch operations also serve take their fused kernel only then."""
+    # (asked first: the compiler folds the answer and traces none of the rest)
+    if torch.compiler.is_compiling():
+        return False
     if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
             or torch._C._functorch.peek_interpreter_stack() is not None
-            or forward_ad._current_level >= 0 or torch.jit.is_tracing()
-            or torch.compiler.is_compiling()):
+            or forward_ad._current_level >= 0 or torch.jit.is_tracing()):
         return False
     grad = torch.is_grad_enabled()
     return all(type(t) in _PLAIN_TYPES and t.is_cuda and not (grad and t.requires_grad)
