@@ -25,6 +25,9 @@ _DTYPES = {torch.bfloat16: 0, torch.float16: 1}
 
 def _takes(x, layers):
     """Whether hb_linear_rows takes rows ``x`` through each (weight, bias) of ``layers``."""
+    # (first: a traced or transformed tensor has no address to look at)
+    if not _lib.is_plain(x, *(t for layer in layers for t in layer if t is not None)):
+        return False
     if x.ndim != 2 or not 1 <= x.shape[0] <= MAX_ROWS or x.dtype not in _DTYPES or x.shape[1] % 8:
         return False
     if x.shape[1] == 0 or x.stride(1) != 1 or x.stride(0) % 8 or not 0 <= x.stride(0) < 2**31 or x.data_ptr() % 16:
@@ -36,7 +39,7 @@ def _takes(x, layers):
             return False
         if any(t is not None and (t.dtype != x.dtype or t.device != x.device) for t in (w, b)):
             return False
-    return _lib.is_plain(x, *(t for layer in layers for t in layer if t is not None))
+    return True
 
 
 def _launch(xs, layers, outs, *, sum=1, silu=False):
