@@ -11,6 +11,7 @@ from pathlib import Path
 
 import torch
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 _PKG = Path(__file__).resolve().parent
 LIB_PATH = _PKG / "libhilberta_hip.so"
@@ -161,12 +162,16 @@ def stream_ptr(device) -> int:
 
 def is_plain(*tensors) -> bool:
     """True for ordinary device tensors outside any transform: no subclass (fake tensors), no
-    dispatch or function mode, tracing or torch.func level, no forward- or reverse-mode gradient.
-    Calls that composed torch operations also serve take their fused kernel only then."""
+    dispatch mode, no function mode but torch's default device (it sets the device of factory calls
+    that name none), no tracing or torch.func level, no forward- or reverse-mode gradient.  Calls that
+    composed torch operations also serve take their fused kernel only then."""
     # (asked first: the compiler folds the answer and traces none of the rest)
     if torch.compiler.is_compiling():
         return False
-    if (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+    modes = torch._C._len_torch_function_stack()
+    if modes and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(modes)):
+        return False
+    if (torch._C._len_torch_dispatch_stack()
             or torch._C._functorch.peek_interpreter_stack() is not None
             or forward_ad._current_level >= 0 or torch.jit.is_tracing()):
         return False

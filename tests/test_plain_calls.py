@@ -7,7 +7,7 @@ import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 
-from hilberta_amd import flux_cond, flux_inputs, sampling_layout
+from hilberta_amd import _lib, flux_cond, flux_inputs, sampling_layout
 
 
 def _rows(gen, *shape):
@@ -64,3 +64,28 @@ def test_fake_tensors(name):
         warnings.simplefilter("error")
         got = call(*(torch.empty(t.shape, dtype=t.dtype) for t in tensors))
     assert [t.shape for t in _flat(got)] == want
+
+
+class _Device(torch.Tensor):
+    """(stands for a device tensor where there is none)"""
+
+    is_cuda = True
+
+
+def test_default_device_is_plain(monkeypatch):
+    """torch.set_default_device is a function mode, and the fused passes are taken under it; under any
+    other, alone or beside it, they are not."""
+    monkeypatch.setattr(_lib, "_PLAIN_TYPES", (_Device,))
+    t = torch.zeros(2).as_subclass(_Device)
+    assert _lib.is_plain(t)
+    with torch.device("cpu"):
+        assert torch._C._len_torch_function_stack() == 1 and _lib.is_plain(t)
+        with torch.overrides.BaseTorchFunctionMode():
+            assert not _lib.is_plain(t)
+    try:
+        torch.set_default_device("cpu")
+        assert _lib.is_plain(t)
+    finally:
+        torch.set_default_device(None)
+    with torch.overrides.BaseTorchFunctionMode(), torch.device("cpu"):
+        assert not _lib.is_plain(t)
