@@ -28,6 +28,9 @@ def _takes(x, layers):
     # (first: a traced or transformed tensor has no address to look at)
     if not _lib.is_plain(x, *(t for layer in layers for t in layer if t is not None)):
         return False
+    # (under autocast the torch calls compute in its type, whatever the layer's)
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != x.dtype:
+        return False
     if x.ndim != 2 or not 1 <= x.shape[0] <= MAX_ROWS or x.dtype not in _DTYPES or x.shape[1] % 8:
         return False
     if x.shape[1] == 0 or x.stride(1) != 1 or x.stride(0) % 8 or not 0 <= x.stride(0) < 2**31 or x.data_ptr() % 16:
