@@ -36,9 +36,7 @@ def _takes(x, layers):
     if x.shape[1] == 0 or x.stride(1) != 1 or x.stride(0) % 8 or not 0 <= x.stride(0) < 2**31 or x.data_ptr() % 16:
         return False
     for w, b in layers:
-        if w.ndim != 2 or w.shape[1] != x.shape[1] or not w.shape[0] or max(w.shape) >= 2**31:
-            return False
-        if not w.is_contiguous() or w.data_ptr() % 16:
+        if w.ndim != 2 or w.shape[1] != x.shape[1] or not w.shape[0] or not w.is_contiguous() or w.data_ptr() % 16:
             return False
         if b is not None and (b.shape != w.shape[:1] or not b.is_contiguous()):
             return False

@@ -26,9 +26,3 @@ def test_autocast_to_another_type(dtype):
     finally:
         torch.set_autocast_enabled("cuda", was[0])
         torch.set_autocast_dtype("cuda", was[1])
-
-
-def test_sizes_past_32_bits():
-    """The kernel's sizes are 32-bit: 2^32 + 8 would arrive as 8.  (Memory is reserved, never touched.)"""
-    x, w = (torch.empty(1, 2**32 + 8, dtype=torch.bfloat16) for _ in range(2))
-    assert not flux_cond._takes(x, [(w, None)])
