@@ -112,6 +112,9 @@ Tensor attention_workspace(at::Device device, int64_t need) {
 std::vector<int64_t> workspace_keys() { return workspaces().keys(); }
 void clear_workspaces() { workspaces().clear(); }
 
+// The C ABI this library was compiled against (ops.py compares it before it binds the operators).
+int64_t abi_version() { return HB_ABI_VERSION; }
+
 // ------------------------------------------------------------------ operators
 struct Shape {
   int32_t batch, heads, tokens, dim, dtype;
@@ -325,6 +328,7 @@ TORCH_LIBRARY(hilberta_hip, m) {
   m.def("_attention_workspace(Device device, int need) -> Tensor");
   m.def("_workspace_keys() -> int[]");
   m.def("_clear_workspaces() -> ()");
+  m.def("_abi_version() -> int");
 }
 
 TORCH_LIBRARY_IMPL(hilberta_hip, CUDA, m) {
@@ -338,6 +342,7 @@ TORCH_LIBRARY_IMPL(hilberta_hip, CompositeExplicitAutograd, m) {
   m.impl("_attention_workspace", attention_workspace);
   m.impl("_workspace_keys", workspace_keys);
   m.impl("_clear_workspaces", clear_workspaces);
+  m.impl("_abi_version", abi_version);
 }
 
 // gather_rows and pair_rows: a differentiated call fails in its backward.

@@ -26,7 +26,7 @@ built library the operators do not exist and every use of one raises.
 import torch
 from torch import Tensor
 
-from ._lib import LIB_PATH, load
+from ._lib import LIB_PATH, header_abi_version, load
 
 _NS = "hilberta_hip"
 TORCH_LIB_PATH = LIB_PATH.with_name("libhilberta_torch.so")
@@ -76,6 +76,12 @@ def _load():
                            "(python -m hilberta_amd.build); there is no CPU fallback")
     load()  # the C ABI library, its version checked, before the operators bind to it
     torch.ops.load_library(str(TORCH_LIB_PATH))
+    version = getattr(getattr(torch.ops, _NS), "_abi_version", None)  # (absent in the oldest ones)
+    built, declared = version() if version else 0, header_abi_version()
+    if built != declared:
+        raise RuntimeError(f"{TORCH_LIB_PATH} was built for {f'ABI {built}' if built else 'an older ABI'} but "
+                           f"include/hilberta_hip.h declares ABI {declared}: rebuild the libraries "
+                           "(python -m hilberta_amd.build)")
     fakes = dict(paired_fwd=_fake_none, sparse_fwd=_fake_none, pair_rows=_fake_pair_rows,
                  gather_rows=_fake_gather_rows)
     for name, fake in fakes.items():

@@ -17,7 +17,7 @@
 extern "C" {
 #endif
 
-#define HB_ABI_VERSION 4
+#define HB_ABI_VERSION 5
 #define HB_DTYPE_BF16 0
 #define HB_DTYPE_F16 1
 
