@@ -208,21 +208,33 @@ def _gemm_rounds(rows, columns):
     return -(-(-(-rows // _TILE) * -(-columns // _TILE)) // _CUS)
 
 
+# Joint rows that a GEMM of a single block takes at once: up to JOINT_ROWS, in multiples of JOINT_STEP.
+_JOINT_ROWS, _JOINT_STEP = 5120, 512
+
+
 def _row_parts(T, shape, columns):
     """How a single block's GEMM of ``columns`` outputs walks joint rows [B, N] of T text and N - T
     image tokens: None for all rows at once, else the (batch, first, end) of each GEMM.
 
-    The text rows are a GEMM of their own unless the joint rows fill fewer rounds of tiles, which
-    decides every shape measured on MI355X (3072-wide model, 512 text rows, joint / split us): with
-    16384 image rows a tie, and the image rows alone fill whole rounds (9216 columns 735 / 659, 12288
-    1037 / 942, 3072 313 / 233, 3072 of depth 12288 1088 / 891); with 4096 the joint rows win where
-    they save the text's round (195 / 225, 66 / 85, 242 / 290) and lose on a tie (12288: 282 / 272);
-    with 1024 likewise (82 / 99, 36 / 47, 116 / 149; 126 / 115)."""
+    Text and image rows of every batch element are GEMMs of their own unless all rows, or the joint rows
+    of one element, fill fewer rounds of tiles and are few and even enough.  Measured on MI355X for the
+    four GEMMs of a 3072-wide model (together, us; text and image apart / as chosen here): 512 + 1024
+    rows 395 / 319, twice 789 / 554, three times 1184 / 734; 512 + 4096 rows 836 / 726, twice 1671 /
+    1452.  Larger row counts gain nothing or lose: 512 + 16384 rows 2575 apart, 3028 joint, twice 5149,
+    5577; twice 512 + 4096 rows all at once 1925.  So do uneven ones, for which the library picks
+    kernels of half the rate (3072 columns of depth 12288: 4096 rows 220 us, 4224 392, 4352 400, 4608
+    228).  Saved rounds alone, without both limits, lost up to 36 % on 54 of 516 shapes of batch 1-4,
+    text of 128-1024 and images of 256-16384 rows; with them none lost."""
     B, N = shape
-    split = B * (_gemm_rounds(T, columns) + _gemm_rounds(N - T, columns))
-    if _gemm_rounds(B * N, columns) < split:
+    apart = _gemm_rounds(T, columns) + _gemm_rounds(N - T, columns)
+
+    def joint(rows, rounds):
+        return rows <= _JOINT_ROWS and rows % _JOINT_STEP == 0 and _gemm_rounds(rows, columns) < rounds
+
+    if joint(B * N, B * apart):
         return None
-    return [(b, lo, hi) for b in range(B) for lo, hi in ((0, T), (T, N))]
+    ranges = ((0, N),) if joint(N, apart) else ((0, T), (T, N))
+    return [(b, lo, hi) for b in range(B) for lo, hi in ranges]
 
 
 def _linear_rows(x, weight, bias, out, T, *, gelu=False, add=None):

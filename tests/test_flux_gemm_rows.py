@@ -24,3 +24,33 @@ def test_every_row_once(batch, T, N, columns):
     out = torch.full((batch, N, columns), float("nan"))
     _linear_rows(x, w, b, out, T, add=(y, w2))
     assert torch.allclose(out, x @ w.t() + b + y @ w2.t(), atol=1e-5)
+
+
+@pytest.mark.parametrize("batch,T,N,columns,parts", [
+    (1, 512, 1536, 8, None), (3, 512, 1536, 8, None), (11, 256, 512, 8, [(0, 512)]), (2, 512, 4608, 8, [(0, 4608)]),
+    (1, 512, 1408, 8, [(0, 512), (512, 1408)]),
+    (2, 1024, 6144, 8, [(0, 1024), (1024, 6144)]), (2, 512, 512, 8, None)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_every_walk(batch, T, N, columns, parts, gelu):
+    """All rows at once, one element at a time, and text and image apart, each with more than one part and
+    with text; the second product and the activation on every one."""
+    assert _row_parts(T, (batch, N), columns) == (
+        None if parts is None else [(b, lo, hi) for b in range(batch) for lo, hi in parts])
+    gen = torch.Generator().manual_seed(N)
+    x, y = torch.randn(batch, N, 2, generator=gen), torch.randn(batch, N, 1, generator=gen)
+    w, b, w2 = (torch.randn(s, generator=gen) for s in ((columns, 2), (columns,), (columns, 1)))
+    out = torch.full((batch, N, columns), float("nan"))
+    _linear_rows(x, w, b, out, T, gelu=gelu, add=None if gelu else (y, w2))
+    ref = x @ w.t() + b
+    ref = torch.nn.functional.gelu(ref, approximate="tanh") if gelu else ref + y @ w2.t()
+    # sums of two or three fp32 products in another order; the CPU epilogue of _addmm_activation may be
+    # the exact GELU, which the tanh form follows to 5e-4
+    assert (out - ref).abs().max() <= (5e-4 if gelu else 1e-5)
+
+
+def test_batches_of_the_measured_shapes():
+    """Batch 2: 1024 px joins each element's rows, never both at once; 2048 px stays apart."""
+    for columns in (9216, 3072):
+        assert _row_parts(512, (2, 4608), columns) == [(0, 0, 4608), (1, 0, 4608)]
+    for columns in (9216, 12288, 3072):
+        assert _row_parts(512, (2, 16896), columns) == [(b, *r) for b in (0, 1) for r in ((0, 512), (512, 16896))]
