@@ -65,9 +65,25 @@ def _launch(xs, layers, outs, *, sum=1, silu=False):
     return outs
 
 
+def _pays(rows, depth, columns, layers):
+    """Whether one launch for ``layers`` layers of ``columns`` outputs in all beats a library call for each.
+
+    With one or two rows it is bound by the read of the weights and always does; with more, by its
+    products, and the library's matrix instructions win past a depth, sooner where fewer columns leave
+    CUs idle (hb_linear_rows' line between one and four columns per wave).  One layer, kernel / library
+    us on MI355X: 18432 columns, 8 rows of depth 6144 75 / 102, of 8192 91 / 71; 9216 columns, 8 rows of
+    depth 1024 20 / 20, of 2048 33 / 20, 4 rows of 3072 25 / 20; 3072 columns, 8 rows of depth 3072
+    17 / 20, of 4096 22 / 20.  All modulations of a two-block 3072-wide model, 8 rows: 101 / 160."""
+    if rows <= 2:
+        return True
+    if columns >= 16384:
+        return depth <= 6144
+    return depth <= 4096 and columns * depth <= 3072 * 3072 * layers
+
+
 def linear_layers(x, layers):
     """[F.linear(x, weight, bias) for weight, bias in layers] for rows x [B, K]."""
-    if not layers or not _takes(x, layers):
+    if not layers or not _takes(x, layers) or not _pays(*x.shape, sum(w.shape[0] for w, _ in layers), len(layers)):
         return [F.linear(x, w, b) for w, b in layers]
     return _launch([x] * len(layers), layers, [x.new_empty(x.shape[0], w.shape[0]) for w, _ in layers])
 
