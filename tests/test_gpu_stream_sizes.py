@@ -65,3 +65,44 @@ def test_gather(hip_device, row_bytes):
     index = torch.randperm(rows, device=hip_device)
     say(f"case gather past the cache size, rows of {row_bytes} bytes")
     assert torch.equal(index_select_rows(x, 0, index), x.index_select(0, index))
+
+
+def _us(call, n=10):
+    """Shortest of five times a call, in microseconds."""
+    best = float("inf")
+    for _ in range(6):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        begin.record()
+        for _ in range(n):
+            call()
+        end.record()
+        torch.cuda.synchronize()
+        best = min(best, begin.elapsed_time(end) / n * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("unique", [1, 16, 16384])
+def test_gather_of_repeated_rows(hip_device, unique):
+    """More rows than the source has, past the line: the same bytes, and (from the caches) in less time
+    than a copy takes that reads as much as it writes."""
+    from hilberta_amd.layout import index_select_rows
+
+    x = torch.randn(unique, 3072, device=hip_device).to(torch.bfloat16)
+    index = torch.randint(0, unique, (65536,), device=hip_device)
+    say(f"case gather of 65536 rows out of {unique}")
+    out = index_select_rows(x, 0, index)
+    assert torch.equal(out, x.index_select(0, index))
+    if unique <= 16:
+        source = torch.empty_like(out)
+        took, copy = _us(lambda: index_select_rows(x, 0, index)), _us(lambda: out.copy_(source))
+        say(f"gather {took:.1f} us, copy {copy:.1f} us")
+        assert took < copy
+
+
+def test_gather_of_one_image_for_a_batch(hip_device):
+    from hilberta_amd.layout import index_select_rows
+
+    x = torch.randn(1, 8192, 3072, device=hip_device).to(torch.bfloat16).expand(4, -1, -1)
+    index = torch.randperm(8192, device=hip_device)
+    say("case gather of an expanded batch")
+    assert torch.equal(index_select_rows(x, 1, index), x.index_select(1, index))
