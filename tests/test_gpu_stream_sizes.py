@@ -106,3 +106,27 @@ def test_gather_of_one_image_for_a_batch(hip_device):
     index = torch.randperm(8192, device=hip_device)
     say("case gather of an expanded batch")
     assert torch.equal(index_select_rows(x, 1, index), x.index_select(1, index))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_adaln_of_repeated_rows(hip_device, dtype):
+    """One image for a batch and one row of y for an image, past the line: as with copies of them."""
+    from hilberta_amd.flux_norm import adaln_modulate
+
+    C, B = 1024, 4
+    rows = CACHE // (2 * C * 4 * B) + 5
+    gen = torch.Generator(hip_device).manual_seed(7)
+    new = lambda *s: torch.randn(*s, device=hip_device, generator=gen).to(dtype)  # noqa: E731
+    x, y = new(1, rows, C).expand(B, -1, -1), new(B, 1, C).expand(-1, rows, -1)
+    shift, scale, gate = new(B, 3 * C).chunk(3, 1)
+    say(f"case adaln of repeated rows past the cache size {dtype}")
+
+    def call(x, y):
+        r = torch.empty(B, rows, C, device=hip_device, dtype=dtype)
+        return r, adaln_modulate(x, shift, scale, y=y, gate=gate, x_out=r)
+
+    dense = call(x.contiguous(), y.contiguous())
+    for pair in ((x, y), (x, y.contiguous()), (x.contiguous(), y)):
+        for got, ref in zip(call(*pair), dense):
+            assert torch.equal(got, ref)
+    assert torch.equal(adaln_modulate(x, shift, scale), adaln_modulate(x.contiguous(), shift, scale))
