@@ -194,6 +194,18 @@ def _linear_into(x, weight, bias, out):
         torch.addmm(bias, x[b], weight.t(), out=out[b])
 
 
+def _linear(x, weight, bias):
+    """F.linear(x, weight, bias) of [B, rows, K].  Rows that are a range of a larger buffer are one GEMM
+    per batch element: of more than one element torch makes a batched product with the transposed
+    weights as its right operand, which has faulted MI355X in bf16, and adds the bias to what that
+    rounded."""
+    if x.is_contiguous():
+        return F.linear(x, weight, bias)
+    out = x.new_empty(*x.shape[:2], weight.shape[0])
+    _linear_into(x, weight, bias, out)
+    return out
+
+
 def _gelu_linear(x, weight, bias):
     """GELU(tanh)(x @ weight^T + bias) with the activation in the GEMM epilogue."""
     flat = x.reshape(-1, x.shape[-1])
@@ -354,8 +366,8 @@ class FluxTransformer:
         self._attend(attention, layer, qk[0], qk[1], v, o)
         del qk, v, qkv
         o = o.view(B, T + n, C)
-        ax = F.linear(o[:, T:], *w["out_x"])
-        ac = F.linear(o[:, :T], *w["out_c"])
+        ax = _linear(o[:, T:], *w["out_x"])
+        ac = _linear(o[:, :T], *w["out_c"])
         del o
         xn, cn = adaln_modulate_pair(dict(x=x, shift=sx2, scale=scx2, y=ax, gate=gx, x_out=x),
                                      dict(x=c, shift=sc2, scale=scc2, y=ac, gate=gc, x_out=c), eps=s.eps)
@@ -444,8 +456,8 @@ class FluxTransformer:
         cos, sin = rotary_tables(torch.cat([txt_ids, img_ids]).to(self.device))
         double_mods, single_mods, out_mods = self._modulations(self.temb(timestep, guidance,
                                                                          pooled_projections, silu=True))
-        x = F.linear(hidden_states.to(self.dtype), *self.x_embedder)
-        c = F.linear(encoder_hidden_states.to(self.dtype), *self.context_embedder)
+        x = _linear(hidden_states.to(self.dtype), *self.x_embedder)
+        c = _linear(encoder_hidden_states.to(self.dtype), *self.context_embedder)
         (sx, scx, *_), (sc, scc, *_) = double_mods[0]
         xn, cn = adaln_modulate_pair(dict(x=x, shift=sx, scale=scx), dict(x=c, shift=sc, scale=scc), eps=s.eps)
         h = torch.empty(B, N, s.hidden, device=x.device, dtype=x.dtype)
@@ -466,7 +478,7 @@ class FluxTransformer:
                                        s.num_layers + j, nxt)
         if hn.shape[1] != n:   # no single blocks: the last double block modulated every row
             hn = hn[:, T:]
-        out = F.linear(hn, *self.proj_out)
+        out = _linear(hn, *self.proj_out)
         if layout is not None and layout_scope == "transformer":
             out = index_select_rows(out, 1, layout.inverse)
         return out

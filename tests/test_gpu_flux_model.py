@@ -144,3 +144,20 @@ def test_full_size_model_parameter_count_and_step(hip_device):
     say(f"  prediction std {float(out.float().std()):.3f}")
     del model
     torch.cuda.empty_cache()
+
+
+def test_batch_equals_its_elements(hip_device, small):
+    """Three images at once: each as alone, up to bf16 rounding order (single-block GEMMs may walk their
+    rows otherwise, conditioning rows are summed otherwise)."""
+    from hilberta_amd.bridge_k import paired_plan_device
+    from hilberta_amd.flux_model import PersistentAttention, synthetic_inputs
+
+    model, _ = small
+    say("case flux model batch 3 vs its elements")
+    attention = PersistentAttention(paired_plan_device(4, 1, grid_size=64, device=hip_device), hip_device)
+    args = synthetic_inputs(hip_device, grid=64, batch=3, shape=model.shape, seed=5)
+    together = model(**args, attention=attention)
+    torch.cuda.synchronize()
+    for b in range(3):
+        one = {k: v if k.endswith("_ids") else v[b:b + 1] for k, v in args.items()}
+        assert _rel(together[b:b + 1], model(**one, attention=attention)) <= REL_L2
