@@ -130,3 +130,22 @@ def test_adaln_of_repeated_rows(hip_device, dtype):
         for got, ref in zip(call(*pair), dense):
             assert torch.equal(got, ref)
     assert torch.equal(adaln_modulate(x, shift, scale), adaln_modulate(x.contiguous(), shift, scale))
+
+
+@pytest.mark.parametrize("expand", [(4, -1, -1), (1, -1, -1)])
+def test_qk_prep_of_one_image_for_a_batch(hip_device, expand):
+    """A batch stride of zero past the line, and a single image at a row stride of its own."""
+    from hilberta_amd.flux_inputs import qk_prep_pair
+
+    heads = 8
+    n = CACHE // (heads * 1024 * expand[0]) + 13
+    gen = torch.Generator(hip_device).manual_seed(8)
+    x = torch.randn(1, n, 3 * heads * 128, device=hip_device, generator=gen).to(torch.bfloat16)
+    x = x[..., :2 * heads * 128].expand(*expand)
+    w = torch.rand(128, device=hip_device, generator=gen).to(torch.bfloat16)
+    cos, sin = torch.rand(2, n, 128, device=hip_device, generator=gen)
+    say(f"case qk_prep of an expanded batch {expand[0]}")
+    got = qk_prep_pair(None, x, heads=heads, cos=cos, sin=sin, weights=((None, w), (None, w)))
+    one = qk_prep_pair(None, x[:1], heads=heads, cos=cos, sin=sin, weights=((None, w), (None, w)))
+    for b in range(expand[0]):
+        assert torch.equal(got[:, b], one[:, 0])
