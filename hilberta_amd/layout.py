@@ -61,6 +61,7 @@ def index_select_rows(x, dim, index, *, out=None, error=None, check=False):
 
 def gather_into(x, dim, index, *, out=None, error=None):
     """The hb_gather_rows launch behind index_select_rows (arguments already checked there)."""
+    index = index.contiguous()   # (the kernel walks it by itself)
     inner = x.shape[dim + 1 :]
     row_elems = math.prod(inner)
     expect = 1
