@@ -79,8 +79,8 @@ def gather_into(x, dim, index, *, out=None, error=None):
         out = torch.empty(shape, dtype=x.dtype, device=x.device)
     elif list(out.shape) != shape or out.dtype != x.dtype or out.device != x.device or not out.is_contiguous():
         raise ValueError("out must be contiguous with the gathered shape and x's dtype, on x's device")
-    if error is not None and (error.dtype != torch.int32 or error.device != x.device or not error.numel()):
-        raise ValueError("error must be an int32 tensor on x's device")
+    if error is not None and (error.device != x.device or error.numel() * error.element_size() < 4):
+        raise ValueError("error must be an int32 scalar on x's device")
     es = x.element_size()
     dst_outer = index.numel() * row_elems
     lib = _lib.load()

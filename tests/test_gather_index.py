@@ -29,7 +29,7 @@ def test_written_tensors_on_the_device():
     """The kernel writes through these addresses: host memory under a device call would fault."""
     x, index = torch.zeros(12, 3), torch.arange(4)
     with patch.object(_lib, "load", side_effect=AssertionError("launched")):
-        for kw in (dict(out=torch.empty(4, 3, device="meta")), dict(error=torch.zeros(1)),
+        for kw in (dict(out=torch.empty(4, 3, device="meta")), dict(error=torch.zeros(1, dtype=torch.int8)),
                    dict(error=torch.zeros(1, dtype=torch.int32, device="meta")),
                    dict(error=torch.zeros(0, dtype=torch.int32))):
             with pytest.raises(ValueError):
