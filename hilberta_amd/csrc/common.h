@@ -27,11 +27,14 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
-// A pass that reads and writes more than the 256 MB last-level cache reads its input past the caches
-// (STREAM): it cannot be there from an earlier pass, and allocating it evicts the output the next
-// kernel reads.  Measured on adaln_kernel with 3072-wide rows, three tensors in turn: 403 MB 78.0 ->
-// 68.6 us, 302 MB 59.0 -> 53.5; below the line the same loads lose whatever the caches still hold (100
-// MB 18.6 -> 21.3 us; one tensor again and again, 246 MB 39.3 -> 44.9).
+// Past a total of 256 MB, the last-level cache's size, a pass reads inputs that it reads once past the
+// caches (STREAM).  The line is on all that it moves, inputs and outputs, and is drawn where streamed
+// loads won when measured: adaln_kernel with 3072-wide rows, three tensors in turn, 403 MB 78.0 -> 68.6
+// us, 302 MB 59.0 -> 53.5; the gather and the Q/K pass at 400-430 MB.  Below it they lose what the caches
+// still hold (100 MB 18.6 -> 21.3 us; one tensor again and again, 246 MB 39.3 -> 44.9), and a little above
+// it they can: an input just written may still be there (one set of tensors again and again, 302 MB 53.2
+// -> 54.3; after the product that writes y 227 -> 225).  Inputs that repeat, by a stride of zero or more
+// gathered rows than there are, are read through the caches at every size.
 constexpr int64_t CACHE_BYTES = 256ll << 20;
 
 template <bool STREAM, typename T>

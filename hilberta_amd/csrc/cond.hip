@@ -21,7 +21,7 @@
 namespace hb {
 namespace {
 
-constexpr int MAX_LAYERS = 64;  // layer descriptors per launch (2.5 KB of kernel arguments)
+constexpr int MAX_LAYERS = 64;  // layer descriptors per launch (48 bytes each: 3 KB of kernel arguments)
 
 struct Layer {
   const uint16_t* x;     // [batch, k], rows x_stride apart

@@ -274,9 +274,9 @@ class FluxTransformer:
     [B, N, 3C] buffer (V is read from it in place), Q and K are normalised and rotated by one
     qk_prep_pair launch, every gated residual add is fused with the following AdaLN modulation
     (flux_norm.adaln_modulate; all blocks' modulation vectors depend only on the timestep
-    embedding and are computed up front, flux_cond.linear_layers), the MLP GELU runs in the GEMM epilogue, and the single
-    blocks' output projection over [attention | mlp] is two accumulating GEMMs instead of a
-    concatenation.
+    embedding and are computed up front, flux_cond.linear_layers), the MLP GELU runs in the GEMM
+    epilogue, and the single blocks' output projection over [attention | mlp] is two accumulating
+    GEMMs instead of a concatenation.
     """
 
     def __init__(self, device, shape: FluxShape = FluxShape(), *, seed=0, dtype=torch.bfloat16):
