@@ -6,7 +6,8 @@
 // double-block stream, 6.4 GB over the 57 blocks.  Bound by the read of the weights.  The library
 // GEMM takes 65 us per 113 MB matrix (1.75 TB/s: a 16 x 16 tile leaves most of the chip idle) and
 // the passes around it about 40 launches of 2-5 us.  Here all modulations of a two-block model,
-// 320 MB, take 53 us (6 TB/s) in one launch, and the embedders three launches.
+// 321 MB, take 52 us (6.2 TB/s) in one launch, of 57 blocks (6.49 GB, two launches) 0.95 ms (6.8 TB/s),
+// and the embedders three launches.  With three to eight rows the products bound it instead.
 //
 //  * linear_rows_kernel: a wave owns ROWS (1 or 4) output columns and reads their weight rows
 //    whole, 16 bytes per lane, with all ROWS loads of a step in flight; the input rows come from L1/L2 and
