@@ -2,7 +2,8 @@
 
 A workspace holds the persistent kernel's work-queue counters (zero-filled once at allocation;
 every launch leaves them at zero) and the partial results of split global query tiles.  Keying
-by stream keeps launches that may overlap in time from sharing one.
+by stream keeps launches that may overlap in time from sharing one; threads of one stream take turns
+in the operators, each until both kernels of its call are enqueued.
 
 A launch captured into a HIP graph gets a workspace of its own, made during the capture with a
 fill kernel (so every replay zero-fills it before the attention kernel runs) and released when the

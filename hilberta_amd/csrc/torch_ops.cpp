@@ -16,6 +16,7 @@
 
 #include <limits>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <tuple>
 #include <utility>
@@ -50,34 +51,48 @@ hipStream_t stream_of(const at::Device& device) {
 // ------------------------------------------------------------------ attention workspaces
 // One workspace per (device, stream): the persistent kernel's work-queue counters (zero-filled once;
 // every launch leaves them at zero) and the partial results of split global query tiles.  Launches
-// that may overlap in time are on different streams and so never share one.  A captured launch gets
-// a workspace of its own from the capture's private pool, zero-filled on every replay.
+// that may overlap in time are on different streams and so never share one.  A call launches two
+// kernels over its workspace, so threads of one stream take turns: each holds the workspace (Lease)
+// until both are enqueued, or the second thread's first kernel could come between them.  A captured
+// launch gets a workspace of its own from the capture's private pool, zero-filled on every replay.
 class Workspaces {
+  struct Held {
+    std::mutex launching;
+    Tensor tensor;
+  };
+
  public:
-  Tensor get(const at::Device& device, int64_t need) {
+  struct Lease {
+    Tensor tensor;
+    std::shared_ptr<Held> held;
+    std::unique_lock<std::mutex> turn;
+  };
+
+  Lease get(const at::Device& device, int64_t need) {
     const auto options = at::TensorOptions().dtype(at::kByte).device(device);
     const int64_t bytes = std::max(need, MIN_WORKSPACE);
     const hipStream_t stream = stream_of(device);
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     TORCH_CHECK(hipStreamIsCapturing(stream, &status) == hipSuccess, "stream capture query failed");
-    if (status != hipStreamCaptureStatusNone) return at::zeros({bytes}, options);
-    const Key key{device.index(), reinterpret_cast<int64_t>(stream)};
+    if (status != hipStreamCaptureStatusNone) return {at::zeros({bytes}, options), nullptr, {}};
+    Lease lease;
     {
-      std::lock_guard<std::mutex> lock(mutex_);
-      const auto it = cache_.find(key);
-      if (it != cache_.end() && it->second.numel() >= need) return it->second;
+      const std::lock_guard<std::mutex> lock(mutex_);
+      std::shared_ptr<Held>& held = cache_[{device.index(), reinterpret_cast<int64_t>(stream)}];
+      if (!held) held = std::make_shared<Held>();
+      lease.held = held;
     }
-    Tensor fresh = at::zeros({bytes}, options);
-    std::lock_guard<std::mutex> lock(mutex_);
-    Tensor& held = cache_[key];
-    if (!held.defined() || held.numel() < need) held = fresh;
-    return held;
+    lease.turn = std::unique_lock<std::mutex>(lease.held->launching);
+    Tensor& tensor = lease.held->tensor;
+    if (!tensor.defined() || tensor.numel() < need) tensor = at::zeros({bytes}, options);
+    lease.tensor = tensor;
+    return lease;
   }
 
   std::vector<int64_t> keys() {
-    std::lock_guard<std::mutex> lock(mutex_);
+    const std::lock_guard<std::mutex> lock(mutex_);
     std::vector<int64_t> out;
-    for (const auto& [key, tensor] : cache_) {
+    for (const auto& [key, held] : cache_) {
       out.push_back(key.first);
       out.push_back(key.second);
     }
@@ -85,15 +100,15 @@ class Workspaces {
   }
 
   void clear() {
-    std::map<Key, Tensor> gone;
-    std::lock_guard<std::mutex> lock(mutex_);
+    std::map<Key, std::shared_ptr<Held>> gone;
+    const std::lock_guard<std::mutex> lock(mutex_);
     gone.swap(cache_);
   }
 
  private:
   using Key = std::pair<int64_t, int64_t>;
   std::mutex mutex_;
-  std::map<Key, Tensor> cache_;
+  std::map<Key, std::shared_ptr<Held>> cache_;
 };
 
 // Never destroyed: at process exit the allocator behind the tensors may be gone first.
@@ -106,7 +121,7 @@ Tensor attention_workspace(at::Device device, int64_t need) {
   TORCH_CHECK_VALUE(device.is_cuda(), "workspaces live on a HIP device");
   if (!device.has_index()) device = at::Device(at::kCUDA, c10::hip::current_device());
   const at::OptionalDeviceGuard guard(device);
-  return workspaces().get(device, need);
+  return workspaces().get(device, need).tensor;
 }
 
 std::vector<int64_t> workspace_keys() { return workspaces().keys(); }
@@ -138,7 +153,7 @@ float* lse_ptr(const std::optional<Tensor>& lse) {
   return lse.has_value() && lse->defined() ? static_cast<float*>(lse->data_ptr()) : nullptr;
 }
 
-Tensor workspace_for(const Tensor& q, const Shape& s, int32_t global_tokens, int32_t width,
+Workspaces::Lease workspace_for(const Tensor& q, const Shape& s, int32_t global_tokens, int32_t width,
                      int32_t key_block, int32_t paired, bool all_queries) {
   const int64_t need = hb_attention_workspace_bytes(s.batch, s.heads, s.tokens, s.dim, global_tokens, width,
                                                     key_block, paired, all_queries);
@@ -153,13 +168,13 @@ void paired_launch(const Tensor& q, const Tensor& k, const Tensor& v, const Tens
   const Shape s = shape_of(q, k, v, out);
   const int32_t width = i32(ids.size(1), "table width"), G = i32(global_tokens, "global_tokens"),
                 kb = i32(key_block, "key_block_size");
-  const Tensor ws = workspace_for(q, s, G, width, kb, 1, all_queries);
+  const auto ws = workspace_for(q, s, G, width, kb, 1, all_queries);
   check(hb_paired_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse_ptr(lse), s.strides, s.batch,
                       s.heads, s.tokens, s.dim, s.dtype, static_cast<const int32_t*>(ids.data_ptr()),
                       static_cast<const int32_t*>(flags.data_ptr()),
                       static_cast<const int32_t*>(counts.data_ptr()), width, G, kb, all_queries,
-                      static_cast<float>(scale_log2), ws.data_ptr(), ws.numel(), i32(num_groups, "num_groups"),
-                      stream_of(q.device())),
+                      static_cast<float>(scale_log2), ws.tensor.data_ptr(), ws.tensor.numel(),
+                      i32(num_groups, "num_groups"), stream_of(q.device())),
         "hb_paired_fwd");
 }
 
@@ -216,11 +231,11 @@ void sparse_fwd(const Tensor& q, const Tensor& k, const Tensor& v, Tensor out, s
     return;
   }
   const int32_t width = i32(ids.size(1), "table width"), G = i32(global_tokens, "global_tokens");
-  const Tensor ws = workspace_for(q, s, G, width, 64, 0, all_queries);
+  const auto ws = workspace_for(q, s, G, width, 64, 0, all_queries);
   check(hb_block_sparse_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse_ptr(lse), s.strides,
                             s.batch, s.heads, s.tokens, s.dim, s.dtype, static_cast<const int32_t*>(ids.data_ptr()),
                             static_cast<const int32_t*>(counts.data_ptr()), width, G, 64, all_queries,
-                            static_cast<float>(scale_log2), ws.data_ptr(), ws.numel(),
+                            static_cast<float>(scale_log2), ws.tensor.data_ptr(), ws.tensor.numel(),
                             i32(num_groups, "num_groups"), stream_of(q.device())),
         "hb_block_sparse_fwd");
 }
