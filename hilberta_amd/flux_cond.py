@@ -5,7 +5,8 @@
 sinusoidal timestep and guidance embeddings and the pooled text, each through a SiLU MLP, summed.
 Both return what the separate torch calls return up to the order of each fp32 sum.  Rows, sizes or
 types the kernels do not take (more than eight rows, depths that are no multiple of 8, other than
-bf16 / fp16, traced or differentiated inputs) run as those torch calls.
+bf16 / fp16, traced or differentiated inputs, autocast to another type) run as those torch calls, and
+so do the layers of ``linear_layers`` that are too deep for their rows (``_pays``).
 """
 
 from __future__ import annotations
