@@ -72,7 +72,8 @@ def _pays(rows, depth, columns, layers):
     With one or two rows it is bound by the read of the weights and always does; with more, by its
     products, and the library's matrix instructions win past a depth, sooner where fewer columns leave
     CUs idle (hb_linear_rows' line between one and four columns per wave).  One layer, kernel / library
-    us on MI355X: 18432 columns, 8 rows of depth 6144 75 / 102, of 8192 91 / 71; 9216 columns, 8 rows of
+    us on MI355X: 18432 columns, 8 rows of depth 6144 75 / 102, of 8192 91 / 71 (of 1024 24 / 20, where a
+    library call is as long as its launch and a second layer turns it); 9216 columns, 8 rows of
     depth 1024 20 / 20, of 2048 33 / 20, 4 rows of 3072 25 / 20; 3072 columns, 8 rows of depth 3072
     17 / 20, of 4096 22 / 20.  All modulations of a two-block 3072-wide model, 8 rows: 101 / 160."""
     if rows <= 2:
